@@ -310,7 +310,7 @@ static EosDev make_eos(const ecg_eos& e) {
   q.eref = e.eref;
   q.mixg = q.sg ? e.gamma * q.pinf / (e.gamma - 1.) : 0.;
   q.mixinv = 1. / (e.gamma - 1.);
-  q.pclamp = -(1. - 1.e-15) * q.pinf + 1.e-15;
+  q.pclamp = q.sg ? -(1. - 1.e-15) * q.pinf + 1.e-15 : 1.e-8;
   q.fg = (float)q.g; q.fpinf = (float)q.pinf; q.fgm1 = (float)q.gm1; q.fgpinf = (float)q.gpinf;
   q.feref = (float)q.eref; q.fmixinv = (float)q.mixinv; q.fpclamp = (float)q.pclamp;
   return q;

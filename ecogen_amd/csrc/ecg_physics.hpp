@@ -32,13 +32,16 @@ enum { BC_NONREFLECTING = 0, BC_WALL = 1, BC_TANK = 2 };
 struct EosDev {
   int sg;          // 1: stiffened gas, 0: ideal gas
   double g;        // gamma
+  // An ideal gas is a stiffened gas of pinf = gpinf = 0: adding or subtracting zero
+  // changes no pressure, so the formulas of both take one form without a select on sg
+  // (the selects cost four instructions per phase of every derived state).
   double pinf;     // SG p_infinity (0 for IG)
   double gm1;      // gamma - 1
   double gpinf;    // gamma * p_infinity
   double eref;
   double mixg;     // gamma*pinf/(gamma-1) (IG: 0)   EosSG.cpp:208-214
   double mixinv;   // 1/(gamma-1)
-  double pclamp;   // SG pressure floor -(1-1e-15)*pinf + 1e-15
+  double pclamp;   // pressure floor: SG -(1-1e-15)*pinf + 1e-15, IG 1e-8
   // The same constants rounded to float (round to nearest, as a conversion on the
   // device rounds): the FP32 kernels read these instead of converting per use.
   float fg, fpinf, fgm1, fgpinf, feref, fmixinv, fpclamp;
@@ -183,6 +186,18 @@ __device__ __forceinline__ double div_ieee(double a, double b, double rb) {
 }
 // A single quotient by the same sequence (no pre-scaling and fix-up steps).
 __device__ __forceinline__ double div1(double a, double b) { return div_ieee(a, b, rcp_ieee(b)); }
+// Quotients by one divisor.
+template <typename R> struct Quot;
+template <> struct Quot<double> {
+  double b, rb;
+  __device__ __forceinline__ explicit Quot(double d) : b(d), rb(rcp_ieee(d)) {}
+  __device__ __forceinline__ double operator()(double a) const { return div_ieee(a, b, rb); }
+};
+template <> struct Quot<float> {
+  float rb;
+  __device__ __forceinline__ explicit Quot(float d) : rb(__builtin_amdgcn_rcpf(d)) {}
+  __device__ __forceinline__ float operator()(float a) const { return a * rb; }
+};
 // The square root as the device's sequence forms it (reciprocal square-root
 // estimate, one Goldschmidt step on the root and its half-reciprocal, two Newton
 // corrections), without the sequence's scaling of arguments below 2^-767 and its
@@ -323,18 +338,18 @@ template <typename R>
 __device__ __forceinline__ R eos_energy(const EosDev& q, R eps, R rho, R p) {
   if constexpr (sizeof(R) == 8) {
     const double rr = dmax<double>(rho, eps);
-    return div_ieee(div_ieee(q.sg ? (p + q.gpinf) : p, q.gm1, q.mixinv), rr, rcp_ieee(rr)) + q.eref;
+    return div_ieee(div_ieee(p + q.gpinf, q.gm1, q.mixinv), rr, rcp_ieee(rr)) + q.eref;
   }
-  return fdiv(fdiv(q.sg ? (p + pv<R>(q.gpinf, q.fgpinf)) : p, pv<R>(q.gm1, q.fgm1)), dmax<R>(rho, eps)) + pv<R>(q.eref, q.feref);
+  return fdiv(fdiv(p + pv<R>(q.gpinf, q.fgpinf), pv<R>(q.gm1, q.fgm1)), dmax<R>(rho, eps)) + pv<R>(q.eref, q.feref);
 }
 template <typename R>
 __device__ __forceinline__ R eos_pressure(const EosDev& q, R rho, R e) {
   R v = pv<R>(q.gm1, q.fgm1) * rho * (e - pv<R>(q.eref, q.feref));
-  return q.sg ? v - pv<R>(q.gpinf, q.fgpinf) : v;
+  return v - pv<R>(q.gpinf, q.fgpinf);
 }
 template <typename R>
 __device__ __forceinline__ R eos_sound(const EosDev& q, R eps, R rho, R p) {
-  return fsqrt(fdiv(pv<R>(q.g, q.fg) * (q.sg ? (p + pv<R>(q.pinf, q.fpinf)) : p), dmax<R>(rho, eps)));
+  return fsqrt(fdiv(pv<R>(q.g, q.fg) * (p + pv<R>(q.pinf, q.fpinf)), dmax<R>(rho, eps)));
 }
 
 // EosSG/EosIG::computeDensityTimesInterfaceSoundSpeedSquare (EosSG.cpp:115-118, EosIG.cpp:113-116)
@@ -351,12 +366,11 @@ __device__ __forceinline__ R eos_p_isentropic(const EosDev& q, R eps, R p0, R rh
   } else {
     base = fpow(fdiv(rhof, dmax<R>(rho0, eps)), pv<R>(q.g, q.fg));
   }
-  return q.sg ? (p0 + pv<R>(q.pinf, q.fpinf)) * base - pv<R>(q.pinf, q.fpinf) : p0 * base;
+  return (p0 + pv<R>(q.pinf, q.fpinf)) * base - pv<R>(q.pinf, q.fpinf);
 }
 template <typename R>
 __device__ __forceinline__ R eos_clamp_p(const EosDev& q, R p) {
-  if (q.sg) return (p <= pv<R>(q.pclamp, q.fpclamp)) ? pv<R>(q.pclamp, q.fpclamp) : p;
-  return (p < R(1.e-8)) ? R(1.e-8) : p;
+  return (p <= pv<R>(q.pclamp, q.fpclamp)) ? pv<R>(q.pclamp, q.fpclamp) : p;
 }
 // Tools::returnNonZeroValue (Tools.cpp:134-145)
 __device__ __forceinline__ double nonzero(double a, double eps) {
@@ -364,13 +378,16 @@ __device__ __forceinline__ double nonzero(double a, double eps) {
   return (double)((0. < a) - (a < 0.)) * eps;
 }
 // computeDensityPfinal (EosSG.cpp:163-170, EosIG.cpp:161-168); FP64 only (relaxation).
-__device__ __forceinline__ double eos_rho_pfinal(const EosDev& q, double eps, double p0, double rho0, double pf,
-                                                 double& drhodp) {
-  double num = q.sg ? q.g * (pf + q.pinf) : q.g * pf;
+__device__ __forceinline__ double eos_rho_pfinal(const EosDev& q, double eps, double p0, double rho0, double pf) {
+  double num = q.g * (pf + q.pinf);
   double denom = num + p0 - pf;
-  double rhof = div1(rho0 * num, q.sg ? nonzero(denom, eps) : dmax(denom, eps));
-  drhodp = div1(rho0 * q.g * (q.sg ? (p0 + q.pinf) : p0), dmax(denom * denom, eps));
-  return rhof;
+  return div1(rho0 * num, q.sg ? nonzero(denom, eps) : dmax(denom, eps));
+}
+// Its derivative d rho / d pf.
+__device__ __forceinline__ double eos_drhodp_pfinal(const EosDev& q, double eps, double p0, double rho0, double pf) {
+  double num = q.g * (pf + q.pinf);
+  double denom = num + p0 - pf;
+  return div1(rho0 * q.g * (p0 + q.pinf), dmax(denom * denom, eps));
 }
 
 // computeDensityHugoniot (EosSG.cpp:152-159, EosIG.cpp:150-157); FP64 only (tank boundary).
@@ -414,11 +431,11 @@ __device__ __forceinline__ R limit(int kind, R s1, R s2) {
     out = (prod > R(1e-9)) ? m : R(0.);
   } else if (kind == LIM_VANLEER) {
     R sum = s1 + s2;
-    if ((fabs(sum) > R(1e-6)) && (prod > R(1e-6))) out = fdiv(R(2.) * prod, sum);
+    if ((fabs(sum) > R(1e-6)) && (prod > R(1e-6))) out = qdiv(R(2.) * prod, sum);
   } else if (kind == LIM_VANALBADA) {
     R sum = s1 + s2;
     if ((fabs(s1) > R(1e-6)) && (fabs(s2) > R(1e-6)) && (fabs(sum) > R(1e-6)) && (prod > R(1e-6)))
-      out = fdiv(prod * sum, s1 * s1 + s2 * s2);
+      out = qdiv(prod * sum, s1 * s1 + s2 * s2);
   } else if (kind == LIM_SUPERBEE) {
     if (prod > R(1e-6)) out = dmax<R>(dmin<R>(R(2.) * fabs(s1), fabs(s2)), dmin<R>(fabs(s1), R(2.) * fabs(s2)));
     if (s1 < R(0.)) out = -out;
@@ -521,8 +538,21 @@ template <int MODEL, int N, typename R>
 __device__ __forceinline__ void derive(const Params& P, Cell<N, R>& s, bool rebuildE) {
   const R eps = pv<R>(P.eps, P.f_eps);
   if (MODEL == M_EULER) {
-    s.e[0] = eos_energy<R>(P.eos[0], eps, s.r[0], s.p[0]);
-    s.c[0] = eos_sound<R>(P.eos[0], eps, s.r[0], s.p[0]);
+    if constexpr (sizeof(R) == 8) {
+      // One reciprocal of the density for the energy and the squared sound speed; the
+      // lean square root inside its range (Euler pressures carry no floor: anything else,
+      // a negative or NaN argument included, takes the library's).
+      const EosDev& q = P.eos[0];
+      const double rr = dmax<double>(s.r[0], eps), ir = rcp_ieee(rr);
+      s.e[0] = div_ieee(div_ieee(s.p[0] + q.gpinf, q.gm1, q.mixinv), rr, ir) + q.eref;
+      const double c2 = div_ieee(q.g * (s.p[0] + q.pinf), rr, ir);
+      double c = sqrt_pos(c2);
+      if (!(c2 > 1.e-200 && c2 < 1.e200)) c = sqrt(c2);
+      s.c[0] = c;
+    } else {
+      s.e[0] = eos_energy<R>(P.eos[0], eps, s.r[0], s.p[0]);
+      s.c[0] = eos_sound<R>(P.eos[0], eps, s.r[0], s.p[0]);
+    }
     if (rebuildE) s.E = s.e[0] + R(0.5) * sqn3<R>(s.u);
     return;
   }
@@ -537,7 +567,7 @@ __device__ __forceinline__ void derive(const Params& P, Cell<N, R>& s, bool rebu
       const EosDev& q = P.eos[k];
       const R ir = __builtin_amdgcn_rcpf(dmax<R>(s.r[k], eps));
       s.e[k] = (s.p[k] + pv<R>(q.gpinf, q.fgpinf)) * pv<R>(q.mixinv, q.fmixinv) * ir + pv<R>(q.eref, q.feref);
-      c2[k] = pv<R>(q.g, q.fg) * (q.sg ? (s.p[k] + pv<R>(q.pinf, q.fpinf)) : s.p[k]) * ir;
+      c2[k] = pv<R>(q.g, q.fg) * (s.p[k] + pv<R>(q.pinf, q.fpinf)) * ir;
       rho += s.a[k] * s.r[k];
       pm += s.a[k] * s.p[k];
     }
@@ -558,8 +588,8 @@ __device__ __forceinline__ void derive(const Params& P, Cell<N, R>& s, bool rebu
   for (int k = 0; k < N; k++) {
     const EosDev& q = P.eos[k];
     const double rr = dmax<double>(s.r[k], eps), ir = rcp_ieee(rr);
-    s.e[k] = div_ieee(div_ieee(q.sg ? (s.p[k] + q.gpinf) : s.p[k], q.gm1, q.mixinv), rr, ir) + q.eref;
-    s.c[k] = sqrt_pos(div_ieee(q.g * (q.sg ? (s.p[k] + q.pinf) : s.p[k]), rr, ir));
+    s.e[k] = div_ieee(div_ieee(s.p[k] + q.gpinf, q.gm1, q.mixinv), rr, ir) + q.eref;
+    s.c[k] = sqrt_pos(div_ieee(q.g * (s.p[k] + q.pinf), rr, ir));
   }
   double rho = 0., pm = 0.;
 #pragma unroll
@@ -707,7 +737,7 @@ __device__ __forceinline__ void hllc_ueq(const Params& P, const Cell<N, R>& Lc, 
       for (int k = 0; k < N; k++) {
         const EosDev& q = P.eos[k];
         const R rks = S.r[k] * ratio;
-        const R pk0 = q.sg ? S.p[k] + pv<R>(q.pinf, q.fpinf) : S.p[k];
+        const R pk0 = S.p[k] + pv<R>(q.pinf, q.fpinf);
         const R pks = pk0 * __builtin_amdgcn_exp2f(pv<R>(q.g, q.fg) * lr) - pv<R>(q.pinf, q.fpinf);
         F.f.alpha[k] = S.a[k] * sM;
         F.f.mass[k] = S.a[k] * rks * sM;
@@ -755,7 +785,7 @@ __device__ __forceinline__ void hllc_ueq(const Params& P, const Cell<N, R>& Lc, 
         }
         base = exp(q.g * lxk);
       }
-      const R pks = q.sg ? (S.p[k] + q.pinf) * base - q.pinf : S.p[k] * base;
+      const R pks = (S.p[k] + q.pinf) * base - q.pinf;
       const R rks_k = rks[k];
       const R eks = eos_energy<R>(q, eps, rks_k, pks);
       F.f.alpha[k] = S.a[k] * sM;
@@ -1153,11 +1183,12 @@ __device__ __forceinline__ void build_prim(const Params& P, Cons<N>& A, Cell<N>&
   if (MODEL == M_EULER) {
     const double m = A.mass[0];
     s.r[0] = m;
-    s.u[0] = A.mom[0] / m; s.u[1] = A.mom[1] / m; s.u[2] = A.mom[2] / m;
+    const double im = rcp_ieee(m);   // one reciprocal for the four quotients by the density
+    s.u[0] = div_ieee(A.mom[0], m, im); s.u[1] = div_ieee(A.mom[1], m, im); s.u[2] = div_ieee(A.mom[2], m, im);
     if (fabs(s.u[0]) < 1.e-8) s.u[0] = 0.;
     if (fabs(s.u[1]) < 1.e-8) s.u[1] = 0.;
     if (fabs(s.u[2]) < 1.e-8) s.u[2] = 0.;
-    s.E = A.energM / m;
+    s.E = div_ieee(A.energM, m, im);
     const double e = s.E - 0.5 * sqn3<double>(s.u);
     s.e[0] = e;
     s.p[0] = eos_pressure<double>(P.eos[0], m, e);
@@ -1200,7 +1231,7 @@ __device__ __forceinline__ void build_prim(const Params& P, Cons<N>& A, Cell<N>&
   // Of the derived state only the mixture density is read afterwards (energy
   // correction); the rest is rebuilt from the stored primitives when needed.
   mixture_density<N>(s);
-  s.E = A.energM / rhoMel;
+  s.E = div_ieee(A.energM, rhoMel, irm);
 }
 
 // alphaNull gate of RelaxationPInfinite::relaxation (RelaxationPInfinite.cpp:51-55):
@@ -1231,18 +1262,26 @@ __device__ __forceinline__ void newton_resume(const Params& P, const Cell<N>& s,
     st.p -= div1(st.f, st.df);
 #pragma unroll
     for (int k = 0; k < N; k++) st.p = eos_clamp_p<double>(P.eos[k], st.p);
-    double f = -1., df = 0.;
+    double f = -1.;
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      double drhodp;
-      rkS[k] = eos_rho_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], st.p, drhodp);
+      rkS[k] = eos_rho_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], st.p);
       akS[k] = div1(s.a[k] * s.r[k], rkS[k]);
-      const double dalpha = div1(s.a[k] * s.r[k] * drhodp, rkS[k] * rkS[k]);
       f += akS[k];
-      df -= dalpha;
     }
     st.f = f;
-    st.df = df;
+    // f' only where another iterate follows: nearly every relaxation is settled by its
+    // first evaluation (1.03 evaluations per relaxation on the 512^3 two-phase case), and
+    // the derivative is two quotients per phase.  A settled st keeps an unread f'.
+    if (fabs(f) > 1e-10) {
+      double df = 0.;
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const double drhodp = eos_drhodp_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], st.p);
+        df -= div1(s.a[k] * s.r[k] * drhodp, rkS[k] * rkS[k]);
+      }
+      st.df = df;
+    }
   } while (fabs(st.f) > 1e-10 && st.it < maxit);
 }
 
@@ -1285,8 +1324,7 @@ __device__ __forceinline__ int relax_end(const Params& P, Cell<N>& s, const Newt
   for (int k = 0; k < N; k++) pI = eos_clamp_p<double>(P.eos[k], pI);
 #pragma unroll
   for (int k = 0; k < N; k++) {
-    double drhodp;
-    const double rho_s = eos_rho_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], pI, drhodp);
+    const double rho_s = eos_rho_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], pI);
     s.a[k] = s.a[k] * s.r[k] / rho_s;
     s.r[k] = rho_s;
     s.p[k] = pI;
@@ -1500,7 +1538,7 @@ __device__ __forceinline__ void correct_and_derive(const Params& P, Cell<N>& s) 
       pp -= s.a[k] * (P.eos[k].mixg * (1. - s.r[k] * 0.) + s.r[k] * P.eos[k].eref);
       denom += s.a[k] * P.eos[k].mixinv * (1. - s.r[k] * 0.);
     }
-    pp /= denom;
+    pp = div1(pp, denom);
 #pragma unroll
     for (int k = 0; k < N; k++) {
       s.p[k] = pp;
