@@ -24,10 +24,10 @@ struct ecg_mlp {
   float* adam_m = nullptr;
   float* adam_v = nullptr;
   float* grad = nullptr;      // reduced gradient
-  float* gpart = nullptr;     // per-block gradient partials
-  float* lpart = nullptr;     // per-block loss partials
-  double* loss_acc = nullptr; // device loss accumulator
-  int gpart_blocks = 0;
+  float* act = nullptr;       // activations of a batch segment, act_ld chunks wide
+  int act_ld = 0;
+  double* loss_acc = nullptr; // per-epoch loss sums (loss_cap of them) and a batch's running sum
+  int loss_cap = 0;
   uint2* frag = nullptr;      // BF16 A fragments (MLP_NFRAG * 64)
   float* bias = nullptr;      // FP32 biases (MLP_NBIAS)
   long long adam_t = 0;

@@ -3,6 +3,7 @@
 // BF16 fragment packing used by the fused MFMA inference in the step kernel.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -12,10 +13,17 @@
 
 namespace ecg {
 
-constexpr int TBS = 64;    // samples per training block (one wave)
-constexpr int LDP = 65;    // padded row of the block's activation matrices
-constexpr int PRM_PAD = (MLP_NPARAM + 3) & ~3;
-constexpr size_t TRAIN_LDS_FLOATS = PRM_PAD + 4 * TBS * LDP + TBS * 13 + 2 * TBS;
+// Training sums run in a fixed order: chunks of TBS samples of a batch, samples in order
+// within a chunk, chunks in order.  A batch is worked off in segments of at most
+// SEG_CHUNKS chunks (35 MB of activations), the running sums carried between them.
+constexpr int TBS = 64;
+constexpr int SEG_CHUNKS = 512;
+constexpr int FB_SAMPLES = 16;             // samples of a k_mlp_fwd_bwd block, of 16 different chunks
+constexpr int LDU = MLP_H + 4;             // padded row of the block's per-sample rows (16-byte aligned)
+// Rows of the activation workspace: row u, sample r of its chunk and chunk c lie at
+// (u * TBS + r) * ld + c, so that a wave whose lanes are chunks reads consecutive words.
+constexpr int ACT_H1 = 0, ACT_DZ2 = MLP_H, ACT_DZ1 = 2 * MLP_H, ACT_P3 = 3 * MLP_H, ACT_X = 4 * MLP_H;
+constexpr int ACT_DY = ACT_X + MLP_IN, ACT_LS = ACT_DY + 1, ACT_ROWS = ACT_LS + 1;
 
 // Orders of the three phase slots; training sees every order of every sample.
 __constant__ int k_slot_perm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
@@ -26,168 +34,230 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
   return z ^ (z >> 31);
 }
 
-// Mean squared error of the clipped remainder r = clip(u) over `count` samples taken
-// as idx = (mult * (q0 + b) + offs) mod n; per-block parameter gradients of
-// inv_batch * sum (y - r)^2 and per-block loss sums.  Every activation matrix
-// of the block (64 samples x 64 units) lives in LDS; each thread owns one
-// sample's row and keeps one row of 64 accumulators in registers.
-__global__ __launch_bounds__(TBS) void k_mlp_fwd_bwd(const float* __restrict__ prm_g, const float* __restrict__ smp,
+// Forward and backward pass of the mean squared error of the clipped remainder
+// r = clip(u), samples idx = (mult * (q0 + b) + offs) mod n of a batch of `count`; every
+// factor of the parameter gradients goes to the activation workspace (rows above).
+// Sixteen threads share a sample, four hidden units each, so that a 4096-record batch
+// fills the chip's 256 CUs with a block each; a thread's sum over the 64 units of a layer
+// stays one chain in the units' order.  Bound by LDS: per unit a 16-byte weight read and a
+// broadcast feed four multiply-adds.  With one thread per sample (64 blocks of one wave,
+// the weight gradients from the same block) a batch took 110 us here and 25 us in the
+// reduction, loss and optimiser kernels behind it; now 12 us and 8 us (k_mlp_grad).
+__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float* __restrict__ prm_g, const float* __restrict__ smp,
                                                      long long n, long long q0, long long count,
                                                      unsigned long long mult, unsigned long long offs,
-                                                     unsigned long long perm_seed, float inv_batch,
-                                                     float* __restrict__ gpart, float* __restrict__ lpart) {
-  extern __shared__ __align__(16) float sm[];
-  float* prm = sm;
-  float* Z1 = prm + PRM_PAD;      // pre-activations of layer 1, later dL/dz1
-  float* H1 = Z1 + TBS * LDP;     // gelu(z1)
-  float* Z2 = H1 + TBS * LDP;     // pre-activations of layer 2
-  float* DZ2 = Z2 + TBS * LDP;    // dL/dz2
-  float* X = DZ2 + TBS * LDP;
-  float* DY = X + TBS * 13;
-  float* LS = DY + TBS;
+                                                     unsigned long long perm_seed, float inv_batch, long long c0,
+                                                     int nchunk, int ld, float* __restrict__ act) {
+  __shared__ __align__(16) float prm[(MLP_NPARAM + 3) & ~3];
+  __shared__ __align__(16) float W2T[MLP_H * LDU];
+  __shared__ __align__(16) float H1[FB_SAMPLES * LDU], PW[FB_SAMPLES * LDU], D2[FB_SAMPLES * LDU], P3[FB_SAMPLES * LDU];
+  __shared__ __align__(16) float X[FB_SAMPLES * MLP_IN];
+  __shared__ float DY[FB_SAMPLES], LS[FB_SAMPLES];
   const int t = threadIdx.x;
-  for (int i = t; i < MLP_NPARAM; i += TBS) prm[i] = prm_g[i];
+  const int s = t >> 4, tj = t & 15;
+  const int r = blockIdx.x & (TBS - 1), cb = (blockIdx.x / TBS) * FB_SAMPLES;
 
-  float x[MLP_IN];
-#pragma unroll
-  for (int i = 0; i < MLP_IN; i++) x[i] = 0.f;
-  float r = 0.f, msk = 0.f;
-  const long long b = (long long)blockIdx.x * TBS + t;
-  if (b < count) {
+  // The sample's record: thread tj < 12 holds input tj, every thread the target.
+  float xin = 0.f, tgt = 0.f, msk = 0.f;
+  const long long b = (c0 + cb + s) * TBS + r;
+  if (cb + s < nchunk && b < count) {
     const unsigned long long q = (unsigned long long)(q0 + b);
     const long long idx = (long long)((mult * q + offs) % (unsigned long long)n);
     const float* rec = smp + idx * SAMPLE_FLOATS;
     const int pm = perm_seed ? (int)(mix64(perm_seed ^ (unsigned long long)idx * 0x9E3779B97F4A7C15ull) % 6ull) : 0;
-#pragma unroll
-    for (int sl = 0; sl < MLP_SLOTS; sl++) {
-      const int src = k_slot_perm[pm][sl];
-#pragma unroll
-      for (int f = 0; f < 4; f++) x[4 * sl + f] = rec[4 * src + f];
-    }
-    r = fminf(fmaxf(rec[14], -MLP_TARGET_CLIP), MLP_TARGET_CLIP);
+    if (tj < MLP_IN) xin = rec[4 * k_slot_perm[pm][tj >> 2] + (tj & 3)];
+    tgt = fminf(fmaxf(rec[14], -MLP_TARGET_CLIP), MLP_TARGET_CLIP);
     msk = 1.f;
   }
-#pragma unroll
-  for (int i = 0; i < MLP_IN; i++) X[t * 13 + i] = x[i];
-  __syncthreads();
-  const float* W1 = prm + MLP_OFF_W1;
-  const float* B1 = prm + MLP_OFF_B1;
-  const float* W2 = prm + MLP_OFF_W2;
-  const float* B2 = prm + MLP_OFF_B2;
-  const float* W3 = prm + MLP_OFF_W3;
-  const float B3 = prm[MLP_OFF_B3];
-  float* z1r = Z1 + t * LDP;
-  float* h1r = H1 + t * LDP;
-  float* z2r = Z2 + t * LDP;
-  float* d2r = DZ2 + t * LDP;
-  float acc[MLP_H];
-
-  // Layer 1.
-#pragma unroll
-  for (int j = 0; j < MLP_H; j++) acc[j] = B1[j];
-#pragma unroll 1
-  for (int i = 0; i < MLP_IN; i++) {
-    const float xi = X[t * 13 + i];
-#pragma unroll
-    for (int j = 0; j < MLP_H; j++) acc[j] += xi * W1[i * MLP_H + j];
-  }
-#pragma unroll
-  for (int j = 0; j < MLP_H; j++) { z1r[j] = acc[j]; h1r[j] = gelu_f(acc[j]); }
-  // Layer 2.
-#pragma unroll
-  for (int j = 0; j < MLP_H; j++) acc[j] = B2[j];
-#pragma unroll 1
-  for (int i = 0; i < MLP_H; i++) {
-    const float hi = h1r[i];
-#pragma unroll
-    for (int j = 0; j < MLP_H; j++) acc[j] += hi * W2[i * MLP_H + j];
-  }
-  // Output and the loss.
-  float y = B3;
-#pragma unroll
-  for (int j = 0; j < MLP_H; j++) { z2r[j] = acc[j]; y += W3[j] * gelu_f(acc[j]); }
-  const float d = y - r;
-  const float loss = msk * d * d;
-  const float dy = msk * 2.f * d * inv_batch;
-  DY[t] = dy;
-  LS[t] = loss;
-#pragma unroll
-  for (int j = 0; j < MLP_H; j++) d2r[j] = dy * W3[j] * gelu_grad_f(acc[j]);
-  // dL/dz1 = (W2 dz2) * gelu'(z1), row by row.
-#pragma unroll
-  for (int i = 0; i < MLP_H; i++) acc[i] = 0.f;
-#pragma unroll 1
-  for (int j = 0; j < MLP_H; j++) {
-    const float gj = d2r[j];
-#pragma unroll
-    for (int i = 0; i < MLP_H; i++) acc[i] += W2[i * MLP_H + j] * gj;
-  }
-#pragma unroll
-  for (int i = 0; i < MLP_H; i++) z1r[i] = acc[i] * gelu_grad_f(z1r[i]);
+  for (int i = t; i < MLP_NPARAM / 4; i += 256)
+    reinterpret_cast<float4*>(prm)[i] = reinterpret_cast<const float4*>(prm_g)[i];
+  if (t < (MLP_NPARAM & 3)) prm[(MLP_NPARAM & ~3) + t] = prm_g[(MLP_NPARAM & ~3) + t];
+  for (int e = t; e < MLP_H * MLP_H; e += 256) W2T[(e & 63) * LDU + (e >> 6)] = prm_g[MLP_OFF_W2 + e];
+  if (tj < MLP_IN) X[s * MLP_IN + tj] = xin;
   __syncthreads();
 
-  // Block sums over the samples (fixed order); one bias / output weight per thread.
-  static_assert(TBS == MLP_H, "one thread per hidden unit in the bias sums");
-  float* gp = gpart + (size_t)blockIdx.x * MLP_NPARAM;
-#pragma unroll 1
-  for (int e = t; e < MLP_H * MLP_H; e += TBS) {
-    const int i = e >> 6, j = e & 63;
-    float a = 0.f;
-    for (int s2 = 0; s2 < TBS; s2++) a += H1[s2 * LDP + i] * DZ2[s2 * LDP + j];
-    gp[MLP_OFF_W2 + e] = a;
-  }
-#pragma unroll 1
-  for (int e = t; e < MLP_IN * MLP_H; e += TBS) {
-    const int i = e >> 6, j = e & 63;
-    float a = 0.f;
-    for (int s2 = 0; s2 < TBS; s2++) a += X[s2 * 13 + i] * Z1[s2 * LDP + j];
-    gp[MLP_OFF_W1 + e] = a;
-  }
-  {
-    float a1 = 0.f, a2 = 0.f, a3 = 0.f;
-    for (int s2 = 0; s2 < TBS; s2++) {
-      a1 += Z1[s2 * LDP + t];
-      a2 += DZ2[s2 * LDP + t];
-      a3 += DY[s2] * gelu_f(Z2[s2 * LDP + t]);
+  const float4* W1 = reinterpret_cast<const float4*>(prm + MLP_OFF_W1) + tj;   // row i: + i * 16
+  const float4* W2 = reinterpret_cast<const float4*>(prm + MLP_OFF_W2) + tj;
+  const float4* WT = reinterpret_cast<const float4*>(W2T) + tj;                // row j: + j * LDU / 4
+  auto unit4 = [&](int off) { return *reinterpret_cast<const float4*>(prm + off + 4 * tj); };
+  auto row4 = [&](float* A) { return reinterpret_cast<float4*>(A + s * LDU); };
+  auto mac = [](float4& a, float x, const float4& w) {
+    a.x += x * w.x; a.y += x * w.y; a.z += x * w.z; a.w += x * w.w;
+  };
+  // A layer's 64 inputs (row in of the sample) against rows w, stride ws, of 64 units.
+  auto layer = [&](float4 acc, const float4* in, const float4* w, int ws) {
+#pragma unroll 8
+    for (int i = 0; i < MLP_H / 4; i++) {
+      const float4 h = in[i];
+      mac(acc, h.x, w[(4 * i + 0) * ws]);
+      mac(acc, h.y, w[(4 * i + 1) * ws]);
+      mac(acc, h.z, w[(4 * i + 2) * ws]);
+      mac(acc, h.w, w[(4 * i + 3) * ws]);
     }
-    gp[MLP_OFF_B1 + t] = a1;
-    gp[MLP_OFF_B2 + t] = a2;
-    gp[MLP_OFF_W3 + t] = a3;
+    return acc;
+  };
+  const float4 w3 = unit4(MLP_OFF_W3);
+
+  float4 z1 = unit4(MLP_OFF_B1);
+#pragma unroll
+  for (int i = 0; i < MLP_IN; i++) mac(z1, X[s * MLP_IN + i], W1[i * (MLP_H / 4)]);
+  row4(H1)[tj] = make_float4(gelu_f(z1.x), gelu_f(z1.y), gelu_f(z1.z), gelu_f(z1.w));
+  __syncthreads();
+  const float4 z2 = layer(unit4(MLP_OFF_B2), row4(H1), W2, MLP_H / 4);
+  const float4 g2 = make_float4(gelu_f(z2.x), gelu_f(z2.y), gelu_f(z2.z), gelu_f(z2.w));
+  row4(PW)[tj] = make_float4(w3.x * g2.x, w3.y * g2.y, w3.z * g2.z, w3.w * g2.w);
+  __syncthreads();
+  float y = prm[MLP_OFF_B3];
+  float4 pw[MLP_H / 4];
+#pragma unroll
+  for (int i = 0; i < MLP_H / 4; i++) pw[i] = row4(PW)[i];
+  __builtin_amdgcn_sched_barrier(0);   // the reads together, then the chain of additions
+#pragma unroll
+  for (int i = 0; i < MLP_H / 4; i++) { y += pw[i].x; y += pw[i].y; y += pw[i].z; y += pw[i].w; }
+  const float d = y - tgt;
+  const float dy = msk * 2.f * d * inv_batch;
+  if (tj == 0) { DY[s] = dy; LS[s] = msk * d * d; }
+  row4(D2)[tj] = make_float4(dy * w3.x * gelu_grad_f(z2.x), dy * w3.y * gelu_grad_f(z2.y), dy * w3.z * gelu_grad_f(z2.z),
+                             dy * w3.w * gelu_grad_f(z2.w));
+  row4(P3)[tj] = make_float4(dy * g2.x, dy * g2.y, dy * g2.z, dy * g2.w);
+  __syncthreads();
+  // dL/dz1 = (W2 dz2) * gelu'(z1), into the output products' rows.
+  const float4 a1 = layer(make_float4(0.f, 0.f, 0.f, 0.f), row4(D2), WT, LDU / 4);
+  row4(PW)[tj] = make_float4(a1.x * gelu_grad_f(z1.x), a1.y * gelu_grad_f(z1.y), a1.z * gelu_grad_f(z1.z),
+                             a1.w * gelu_grad_f(z1.w));
+  __syncthreads();
+
+  // To the workspace, the block's 16 chunks (64 bytes) of one row per four threads.
+  const int u = t >> 2, q4 = 4 * (t & 3);
+  auto put = [&](int row, const float* A, int lda, int col) {
+    *reinterpret_cast<float4*>(act + ((size_t)row * TBS + r) * ld + cb + q4) =
+        make_float4(A[q4 * lda + col], A[(q4 + 1) * lda + col], A[(q4 + 2) * lda + col], A[(q4 + 3) * lda + col]);
+  };
+  put(ACT_H1 + u, H1, LDU, u);
+  put(ACT_DZ2 + u, D2, LDU, u);
+  put(ACT_DZ1 + u, PW, LDU, u);
+  put(ACT_P3 + u, P3, LDU, u);
+  if (u < MLP_IN) put(ACT_X + u, X, MLP_IN, u);
+  else if (u == MLP_IN) put(ACT_DY, DY, 1, 0);
+  else if (u == MLP_IN + 1) put(ACT_LS, LS, 1, 0);
+}
+
+// Parameter gradients of a segment of nchunk chunks from the activation workspace, and
+// with last and adam_m the optimiser step: one wave for eight parameters, a 2 x 4 tile of
+// a weight matrix or eight column sums (and one wave for b3 and the loss).  Lanes are chunks
+// and sum their 64 samples in order; eight threads then add the chunks in order.  633 waves
+// over the chip; a 2 x 4 tile reads six rows for eight products, which keeps a CU's loads
+// (48 cycles of L1 a sample for its two or three waves) below their arithmetic (64 cycles a
+// SIMD).  The eight XCDs take eight rows of W2 each, so that each L2 holds an eighth of h1.
+constexpr int GR_W2 = (MLP_H / 2) * (MLP_H / 4), GR_W1 = (MLP_IN / 2) * (MLP_H / 4), GR_SUM = 3 * MLP_H / 8;
+constexpr int GR_BLOCKS = GR_W2 + GR_W1 + GR_SUM + 1;
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_mlp_grad(const float* __restrict__ act, int nchunk, int ld, int first, int last,
+                                                 float* __restrict__ grad, float* __restrict__ adam_m,
+                                                 float* __restrict__ adam_v, float* __restrict__ prm, float lr_t,
+                                                 double* __restrict__ loss_part, double* __restrict__ loss, int loss_first) {
+  constexpr int LDG = 68, RB = 16;
+  __shared__ __align__(16) float part[8 * LDG];
+  const int t = threadIdx.x, blk = blockIdx.x;
+  int ra, rb, kind, p = -1;   // first rows; 0: tile, 1: column sums, 2: b3 and the loss; the thread's parameter
+  if (blk < GR_W2) {
+    const int i = 2 * ((blk & 7) * 4 + ((blk >> 3) & 3)), j = 4 * (blk >> 5);
+    kind = 0; ra = ACT_H1 + i; rb = ACT_DZ2 + j;
+    p = MLP_OFF_W2 + (i + (t >> 2)) * MLP_H + j + (t & 3);
+  } else if (blk < GR_W2 + GR_W1) {
+    const int e = blk - GR_W2, i = 2 * (e >> 4), j = 4 * (e & 15);
+    kind = 0; ra = ACT_X + i; rb = ACT_DZ1 + j;
+    p = MLP_OFF_W1 + (i + (t >> 2)) * MLP_H + j + (t & 3);
+  } else if (blk < GR_W2 + GR_W1 + GR_SUM) {
+    const int e = blk - GR_W2 - GR_W1, j = 8 * (e & 7);
+    kind = 1; ra = rb = ((e >> 3) == 0 ? ACT_DZ1 : (e >> 3) == 1 ? ACT_DZ2 : ACT_P3) + j;
+    p = ((e >> 3) == 0 ? MLP_OFF_B1 : (e >> 3) == 1 ? MLP_OFF_B2 : MLP_OFF_W3) + j + t;
+  } else {
+    kind = 2; ra = rb = ACT_DY;   // and the losses, the row behind it
+    p = MLP_OFF_B3;
   }
-  if (t == 0) {
-    float a = 0.f, l = 0.f;
-    for (int s2 = 0; s2 < TBS; s2++) { a += DY[s2]; l += LS[s2]; }
-    gp[MLP_OFF_B3] = a;
-    lpart[blockIdx.x] = l;
+  const bool owner = t < ((kind == 2) ? 1 : 8);
+  const bool step = owner && last && adam_m != nullptr;
+  float g = (owner && !first) ? grad[p] : 0.f;
+  float m = 0.f, v = 0.f, w = 0.f;
+  if (step) { m = adam_m[p]; v = adam_v[p]; w = prm[p]; }
+  double lsum = (kind == 2 && t == 1 && !first) ? *loss_part : 0.;
+
+  const size_t rs = (size_t)TBS * ld;
+  for (int c0 = 0; c0 < nchunk; c0 += 64) {
+    const int nc = (nchunk - c0 < 64) ? nchunk - c0 : 64;
+    const float* A = act + ra * rs + c0 + (t < nc ? t : nc - 1);
+    const float* B = act + rb * rs + c0 + (t < nc ? t : nc - 1);
+    float a[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) a[k] = 0.f;
+    // Loads of RB samples are issued together, ahead of the sums (the workspace comes from the
+    // other XCDs' writes; the compiler's own order waited for every load, 24 us).
+    if (kind == 0) {
+      for (int r0 = 0; r0 < TBS; r0 += RB) {
+        float f[RB][6];
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+          const int o = (r0 + r) * ld;
+          f[r][0] = A[o]; f[r][1] = A[rs + o];
+#pragma unroll
+          for (int k = 0; k < 4; k++) f[r][2 + k] = B[k * rs + o];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+          for (int k = 0; k < 8; k++) a[k] += f[r][k >> 2] * f[r][2 + (k & 3)];
+      }
+    } else {
+      const int rows = (kind == 1) ? 8 : 2;
+      for (int r0 = 0; r0 < TBS; r0 += RB) {
+        float f[RB][8];
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+          for (int k = 0; k < 8; k++) f[r][k] = A[(k < rows ? k : 0) * rs + (r0 + r) * ld];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+          for (int k = 0; k < 8; k++) a[k] += f[r][k];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; k++) part[k * LDG + t] = a[k];
+    __syncthreads();
+    if (owner) {
+      const float* q = part + t * LDG;
+      int c = 0;
+      if (nc == 64) {
+        float4 f[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) f[k] = reinterpret_cast<const float4*>(q)[k];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 16; k++) { g += f[k].x; g += f[k].y; g += f[k].z; g += f[k].w; }
+        c = 64;
+      }
+      for (; c < nc; c++) g += q[c];
+    } else if (kind == 2 && t == 1) {
+      for (int c = 0; c < nc; c++) lsum += (double)part[LDG + c];
+    }
   }
-}
-
-// Fixed-order sum of the block partials (deterministic gradients).
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ gpart, int nblk, float* __restrict__ grad) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
-  float s = 0.f;
-  for (int b = 0; b < nblk; b++) s += gpart[(size_t)b * MLP_NPARAM + p];
-  grad[p] = s;
-}
-
-__global__ void k_mlp_loss(const float* __restrict__ lpart, int nblk, double* __restrict__ acc) {
-  if (threadIdx.x != 0) return;
-  double s = 0.;
-  for (int b = 0; b < nblk; b++) s += (double)lpart[b];
-  *acc += s;
-}
-
-__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ prm, const float* __restrict__ grad,
-                                                  float* __restrict__ m, float* __restrict__ v, float lr_t) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
-  const float g = grad[p];
-  const float mm = 0.9f * m[p] + 0.1f * g;
-  const float vv = 0.999f * v[p] + 0.001f * g * g;
-  m[p] = mm;
-  v[p] = vv;
-  prm[p] -= lr_t * mm / (sqrtf(vv) + 1e-8f);
+  if (kind == 2 && t == 1) {
+    if (!last) *loss_part = lsum;
+    else if (loss_first) *loss = lsum;
+    else *loss += lsum;
+  }
+  if (step) {
+    m = 0.9f * m + 0.1f * g;
+    v = 0.999f * v + 0.001f * g * g;
+    adam_m[p] = m;
+    adam_v[p] = v;
+    prm[p] = w - lr_t * m / (sqrtf(v) + 1e-8f);
+  } else if (owner) {
+    grad[p] = g;
+  }
 }
 
 // BF16 A fragments of v_mfma_f32_16x16x16bf16_1k (lane l holds A[l%16][4*(l/16)+j])
@@ -347,7 +417,6 @@ ecg_mlp* ecg_mlp_create(uint64_t seed) {
   ok = ok && hipMalloc(&M->adam_m, MLP_NPARAM * sizeof(float)) == hipSuccess;
   ok = ok && hipMalloc(&M->adam_v, MLP_NPARAM * sizeof(float)) == hipSuccess;
   ok = ok && hipMalloc(&M->grad, MLP_NPARAM * sizeof(float)) == hipSuccess;
-  ok = ok && hipMalloc(&M->loss_acc, sizeof(double)) == hipSuccess;
   ok = ok && hipMalloc(&M->frag, MLP_NFRAG * 64 * sizeof(uint2)) == hipSuccess;
   ok = ok && hipMalloc(&M->bias, MLP_NBIAS * sizeof(float)) == hipSuccess;
   if (!ok) {
@@ -383,7 +452,7 @@ int ecg_mlp_destroy(ecg_mlp* M) {
   if (M->attached > 0) return api_fail(ECG_E_ARG, "the network is the warm start of a solver context (detach it first)");
   if (M->stream) hipStreamSynchronize(M->stream);
   hipFree(M->prm); hipFree(M->adam_m); hipFree(M->adam_v); hipFree(M->grad);
-  hipFree(M->gpart); hipFree(M->lpart); hipFree(M->loss_acc); hipFree(M->frag); hipFree(M->bias);
+  hipFree(M->act); hipFree(M->loss_acc); hipFree(M->frag); hipFree(M->bias);
   if (M->stream) hipStreamDestroy(M->stream);
   delete M;
   return ECG_OK;
@@ -416,30 +485,41 @@ int ecg_mlp_get_params(ecg_mlp* M, float* host) {
   return ECG_OK;
 }
 
-static int ensure_partials(ecg_mlp* M, int nblk) {
-  if (nblk <= M->gpart_blocks) return ECG_OK;
-  HIPCHK(hipStreamSynchronize(M->stream));
-  hipFree(M->gpart);
-  hipFree(M->lpart);
-  M->gpart = nullptr;
-  M->lpart = nullptr;
-  M->gpart_blocks = 0;
-  HIPCHK(hipMalloc(&M->gpart, (size_t)nblk * MLP_NPARAM * sizeof(float)));
-  HIPCHK(hipMalloc(&M->lpart, (size_t)nblk * sizeof(float)));
-  M->gpart_blocks = nblk;
+// Workspace of a batch of nblk chunks and of nloss loss sums.
+static int ensure_workspace(ecg_mlp* M, long long nblk, int nloss) {
+  const int ld = (int)((std::min<long long>(nblk, SEG_CHUNKS) + FB_SAMPLES - 1) / FB_SAMPLES * FB_SAMPLES);
+  if (ld > M->act_ld) {
+    HIPCHK(hipStreamSynchronize(M->stream));
+    hipFree(M->act);
+    M->act = nullptr;
+    M->act_ld = 0;
+    HIPCHK(hipMalloc(&M->act, (size_t)ACT_ROWS * TBS * ld * sizeof(float)));
+    M->act_ld = ld;
+  }
+  if (nloss > M->loss_cap) {
+    HIPCHK(hipStreamSynchronize(M->stream));
+    hipFree(M->loss_acc);
+    M->loss_acc = nullptr;
+    M->loss_cap = 0;
+    HIPCHK(hipMalloc(&M->loss_acc, (size_t)(nloss + 1) * sizeof(double)));   // the last one: a batch's running sum
+    M->loss_cap = nloss;
+  }
   return ECG_OK;
 }
 
-static int launch_fwd_bwd(ecg_mlp* M, const ecg_samples* S, long long n, long long q0, long long count,
-                          unsigned long long mult, unsigned long long offs, unsigned long long perm_seed,
-                          float inv_batch, int nblk) {
-  const size_t lds = TRAIN_LDS_FLOATS * sizeof(float);
-  HIPCHK(hipFuncSetAttribute((const void*)k_mlp_fwd_bwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(nblk), dim3(TBS), lds, M->stream, M->prm, S->buf, n, q0, count, mult,
-                     offs, perm_seed, inv_batch, M->gpart, M->lpart);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, M->stream, M->gpart, nblk, M->grad);
-  hipLaunchKernelGGL(k_mlp_loss, dim3(1), dim3(64), 0, M->stream, M->lpart, nblk, M->loss_acc);
+// Gradient of one batch (nblk chunks) into M->grad, or with adam the optimiser step on it;
+// the batch's loss sum is added to loss sum `e` (set, when loss_first).
+static int launch_batch(ecg_mlp* M, const ecg_samples* S, long long n, long long q0, long long count,
+                        unsigned long long mult, unsigned long long offs, unsigned long long perm_seed,
+                        float inv_batch, long long nblk, bool adam, float lr_t, int e, bool loss_first) {
+  for (long long c0 = 0; c0 < nblk; c0 += SEG_CHUNKS) {
+    const int nc = (int)std::min<long long>(nblk - c0, SEG_CHUNKS);
+    hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(TBS * ((nc + FB_SAMPLES - 1) / FB_SAMPLES)), dim3(256), 0, M->stream, M->prm,
+                       S->buf, n, q0, count, mult, offs, perm_seed, inv_batch, c0, nc, M->act_ld, M->act);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(GR_BLOCKS), dim3(64), 0, M->stream, M->act, nc, M->act_ld, c0 == 0 ? 1 : 0,
+                       c0 + nc >= nblk ? 1 : 0, M->grad, adam ? M->adam_m : (float*)nullptr, M->adam_v, M->prm, lr_t,
+                       M->loss_acc + M->loss_cap, M->loss_acc + e, loss_first ? 1 : 0);
+  }
   HIPCHK(hipGetLastError());
   return ECG_OK;
 }
@@ -449,11 +529,10 @@ int ecg_mlp_gradient(ecg_mlp* M, ecg_samples* S, int64_t n, float* grad, double*
   const long long have = samples_count(S);
   if (have < 0) return api_fail(ECG_E_HIP, "reading the sample counter failed");
   if (n > have) return api_fail(ECG_E_ARG, "more records requested than the buffer holds");
-  const int nblk = (int)((n + TBS - 1) / TBS);
-  int rc = ensure_partials(M, nblk);
+  const long long nblk = (n + TBS - 1) / TBS;
+  int rc = ensure_workspace(M, nblk, 1);
   if (rc != ECG_OK) return rc;
-  HIPCHK(hipMemsetAsync(M->loss_acc, 0, sizeof(double), M->stream));
-  rc = launch_fwd_bwd(M, S, n, 0, n, 1ull, 0ull, 0ull, 1.f / (float)n, nblk);
+  rc = launch_batch(M, S, n, 0, n, 1ull, 0ull, 0ull, 1.f / (float)n, nblk, false, 0.f, 0, true);
   if (rc != ECG_OK) return rc;
   double acc = 0.;
   HIPCHK(hipMemcpyAsync(grad, M->grad, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, M->stream));
@@ -477,7 +556,7 @@ int ecg_mlp_train(ecg_mlp* M, ecg_samples* S, int epochs, int batch, float lr, u
   if (n >= (1ll << 31)) return api_fail(ECG_E_ARG, "at most 2^31 samples per training call");
   if (M->attached > 0) HIPCHK(hipDeviceSynchronize());
   const int nblk = batch / TBS;
-  int rc = ensure_partials(M, nblk);
+  int rc = ensure_workspace(M, nblk, epochs);
   if (rc != ECG_OK) return rc;
   const long long nb = n / batch;
   // Multipliers of the per-epoch affine permutation of the sample order (coprime with n).
@@ -492,23 +571,19 @@ int ecg_mlp_train(ecg_mlp* M, ecg_samples* S, int epochs, int batch, float lr, u
     unsigned long long z = seed * 0x9E3779B97F4A7C15ull + (unsigned long long)e * 0xD1B54A32D192ED03ull + 1ull;
     z = (z ^ (z >> 31)) * 0xBF58476D1CE4E5B9ull;
     const unsigned long long offs = (z ^ (z >> 29)) % (unsigned long long)n;
-    HIPCHK(hipMemsetAsync(M->loss_acc, 0, sizeof(double), M->stream));
     for (long long b = 0; b < nb; b++) {
-      rc = launch_fwd_bwd(M, S, n, b * batch, batch, mult, offs, z | 1ull, 1.f / (float)batch, nblk);
-      if (rc != ECG_OK) return rc;
       M->adam_t++;
       const double bc1 = 1. - std::pow(0.9, (double)M->adam_t);
       const double bc2 = 1. - std::pow(0.999, (double)M->adam_t);
       const float lr_t = (float)(lr * std::sqrt(bc2) / bc1);
-      hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, M->stream, M->prm, M->grad,
-                         M->adam_m, M->adam_v, lr_t);
+      rc = launch_batch(M, S, n, b * batch, batch, mult, offs, z | 1ull, 1.f / (float)batch, nblk, true, lr_t, e, b == 0);
+      if (rc != ECG_OK) return rc;
     }
-    HIPCHK(hipGetLastError());
-    double acc = 0.;
-    HIPCHK(hipMemcpyAsync(&acc, M->loss_acc, sizeof(double), hipMemcpyDeviceToHost, M->stream));
-    HIPCHK(hipStreamSynchronize(M->stream));
-    if (epoch_loss) epoch_loss[e] = acc / (double)(nb * batch);
   }
+  std::vector<double> acc((size_t)epochs);
+  HIPCHK(hipMemcpyAsync(acc.data(), M->loss_acc, sizeof(double) * epochs, hipMemcpyDeviceToHost, M->stream));
+  HIPCHK(hipStreamSynchronize(M->stream));
+  for (int e = 0; e < epochs && epoch_loss; e++) epoch_loss[e] = acc[e] / (double)(nb * batch);
   return mlp_pack(M);
 }
 

@@ -94,6 +94,27 @@ def test_training_gradient_matches_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 65, 1023, 1025, 4160, 32768, 32769, 70001])
+def test_gradient_at_chunk_and_segment_edges(n):
+    """Partial chunks (64 records), partial groups of 16 chunks, lane groups of 64 chunks and
+    segments of 512 chunks.  The bound: a chain of 64 products per unit, twice, and one sum of
+    at most 64 + 1094 float additions (each 6e-8), so 1e-4 of the gradient's norm."""
+    from ecogen_amd import Mlp, Samples
+    rng = np.random.default_rng(n)
+    rec = _random_records(rng, min(n, 2000))
+    rec = rec[rng.integers(0, len(rec), size=n)]
+    prm = rng.normal(0, 0.2, mo.N_PARAM).astype(np.float32)
+    smp = Samples(n)
+    smp.upload(rec)
+    m = Mlp(seed=5)
+    m.set_params(prm)
+    g, loss = m.gradient(smp, n)
+    loss_o, g_o = mo.loss_and_grad(prm.astype(np.float64), rec.astype(np.float64))
+    assert abs(loss - loss_o) <= 1e-4 * loss_o
+    assert np.linalg.norm(g - g_o) <= 1e-4 * np.linalg.norm(g_o)
+
+
+@pytest.mark.gpu
 def test_mfma_inference_matches_bf16_oracle():
     from ecogen_amd import Mlp, Samples
     print("[learned] inference", flush=True)
