@@ -1190,36 +1190,41 @@ static int noalloc_scratch(unsigned char** out) {
   return ECG_OK;
 }
 
-// Zeroed counter slots (dtMax slots at 1e10), zeroed warning counter, the given clock.
-__global__ void k_noalloc_reset(Clock* clk, Counters* cnt, unsigned long long* warn_cnt, Clock v) {
+// Everything a step on caller buffers finds in the scratch array, in one launch: the
+// parameter copy, zeroed counter slots (dtMax slots at 1e10), the zeroed warning counter,
+// the given clock (block 0) and the distance tables of the interior faces, the same
+// arithmetic as the host's.  Bound by latency alone: as a host copy and two kernels it
+// took three dependent submissions ahead of every step.
+__global__ __launch_bounds__(256) void k_noalloc_open(Params P, Params* pdev, Clock* clk, Counters* cnt,
+                                                      unsigned long long* warn_cnt, Clock v, double* tab, int64_t o0,
+                                                      int64_t o1, int64_t o2) {
   const int l = threadIdx.x;
-  if (l < ATOMIC_SLOTS) {
-    Counters z = {};
-    z.dtmax_bits = (uint64_t)__double_as_longlong(1.e10);
-    cnt[l] = z;
+  if (blockIdx.x == 0) {
+    constexpr int PW = sizeof(Params) / sizeof(uint64_t);
+    static_assert(sizeof(Params) % sizeof(uint64_t) == 0, "the parameters are copied in 8-byte words");
+    const uint64_t* src = reinterpret_cast<const uint64_t*>(&P);
+    for (int i = l; i < PW; i += 256) reinterpret_cast<uint64_t*>(pdev)[i] = src[i];
+    if (l < ATOMIC_SLOTS) {
+      Counters z = {};
+      z.dtmax_bits = (uint64_t)__double_as_longlong(1.e10);
+      cnt[l] = z;
+    }
+    if (l == 0) {
+      v.fatal = 0;
+      v.fatal_seen = 0;
+      *clk = v;
+      *warn_cnt = 0ull;
+    }
   }
-  if (l == 0) {
-    v.fatal = 0;
-    v.fatal_seen = 0;
-    *clk = v;
-    *warn_cnt = 0ull;
-  }
-}
-
-// Distance tables of the interior faces, the same arithmetic as the host's.
-__global__ void k_dist_tables(double* tab, int nx, int ny, int nz, double dx, double dy, double dz, int64_t o0,
-                              int64_t o1, int64_t o2) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int n3[3] = {nx, ny, nz};
-  const double d3[3] = {dx, dy, dz};
+  const int n3[3] = {P.nx, P.ny, P.nz};
   const int64_t base[3] = {o0, o1, o2};
-  int64_t r = g;
+  int64_t r = (int64_t)blockIdx.x * 256 + l;
+#pragma unroll
   for (int a = 0; a < 3; a++) {
     const int64_t nf = n3[a] > 1 ? n3[a] - 1 : 1;
-    if (r < 3 * nf) {
+    if (r >= 0 && r < 3 * nf) {
       const int k = (int)(r / nf), m = (int)(r % nf);
-      tab[base[a] + r] = (m + 1 < n3[a]) ? face_distance(d3[a], m, k) : 0.;
-      return;
+      tab[base[a] + r] = (m + 1 < n3[a]) ? face_distance(P.d[a], m, k) : 0.;
     }
     r -= 3 * nf;
   }
@@ -1273,12 +1278,10 @@ int ecg_step_noalloc(const ecg_config* cfg, const void* state_in, void* state_ou
   P.warn_cap = 0;
   Clock* clk = reinterpret_cast<Clock*>(S + o_clk);
   Counters* cnt = reinterpret_cast<Counters*>(S + o_cnt);
-  HIPCHK(hipMemcpyAsync(S + o_par, &P, sizeof(Params), hipMemcpyHostToDevice, st));
   const int64_t ntab = (int64_t)Ly.ntab;
-  hipLaunchKernelGGL(k_dist_tables, dim3((unsigned)((ntab + 255) / 256)), dim3(256), 0, st, tab, g.nx, g.ny, g.nz,
-                     P.d[0], P.d[1], P.d[2], (int64_t)Ly.tab_off[0][0], (int64_t)Ly.tab_off[1][0],
-                     (int64_t)Ly.tab_off[2][0]);
-  hipLaunchKernelGGL(k_noalloc_reset, dim3(1), dim3(64), 0, st, clk, cnt, P.warn_cnt, fresh_clock(dt, 0, INFINITY));
+  hipLaunchKernelGGL(k_noalloc_open, dim3((unsigned)((ntab + 255) / 256)), dim3(256), 0, st, P,
+                     reinterpret_cast<Params*>(S + o_par), clk, cnt, P.warn_cnt, fresh_clock(dt, 0, INFINITY), tab,
+                     (int64_t)Ly.tab_off[0][0], (int64_t)Ly.tab_off[1][0], (int64_t)Ly.tab_off[2][0]);
   StepLaunch L;
   std::memset(&L, 0, sizeof(L));
   L.pdev = reinterpret_cast<const Params*>(S + o_par);
@@ -1303,22 +1306,23 @@ int ecg_step_noalloc(const ecg_config* cfg, const void* state_in, void* state_ou
     tank();
     step(P, L, clk, cnt, st);
   }
-  launch_clock(clk, cnt, g.cfl, st);
   HIPCHK(hipGetLastError());
-  Clock hk;
+  // The caller keeps the time: of the clock's bookkeeping only dtMax is left, the least of
+  // the slots (non-negative doubles order as integers), taken here from the one copy.
   Counters hc[ATOMIC_SLOTS];
-  HIPCHK(hipMemcpyAsync(&hk, clk, sizeof(Clock), hipMemcpyDeviceToHost, st));
   HIPCHK(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
   Counters zero, sum;
   std::memset(&zero, 0, sizeof(zero));
   std::memset(&sum, 0, sizeof(sum));
+  uint64_t dtb = UINT64_MAX;
   for (int q = 0; q < ATOMIC_SLOTS; q++) {
     sum.tank_fail += hc[q].tank_fail;
     sum.nonfinite += hc[q].nonfinite;
     sum.newton_warn += hc[q].newton_warn;
+    dtb = std::min(dtb, hc[q].dtmax_bits);
   }
-  if (dtmax_out) *dtmax_out = hk.dt_max;
+  if (dtmax_out) std::memcpy(dtmax_out, &dtb, sizeof(dtb));
   return step_outcome(zero, sum);
 }
 
