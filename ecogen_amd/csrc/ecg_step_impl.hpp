@@ -45,15 +45,32 @@ constexpr int LK_FULL = -2;
 // differences within a dozen steps.
 template <typename R, int LK> constexpr bool crpow() { return LK == LK_FULL && sizeof(R) == 8; }
 
-template <int D, int ES> struct Tile;
-template <int ES> struct Tile<1, ES> { static constexpr int X = 256, Y = 1, Z = 1; };
-template <int ES> struct Tile<2, ES> { static constexpr int X = 16, Y = 16, Z = 1; };
+//
+// Small meshes in 2D and 3D take tiles of 64 cells (8 x 8 and 4 x 4 x 4), one block's
+// waves split over the axes: 128 threads per axis evaluate all its slopes (at most 112),
+// then all its fluxes (at most 80), the axes side by side, and the first wave updates the
+// cells.  A stage's chain is then one slope, one flux and one update instead of two slopes
+// and two fluxes per axis and the update, on four times the blocks (step_small).
+//
+// The tile shape is named by TK: the element size, plus SMALL_TILE for the small tiles.
+constexpr int SMALL_TILE = 64;
+constexpr int tile_esize(int tk) { return tk & 63; }
+constexpr bool tile_small(int tk) { return tk >= SMALL_TILE; }
+template <int D, int TK> struct Tile;
+template <int TK> struct Tile<1, TK> { static constexpr int X = 256, Y = 1, Z = 1; };
+template <int TK> struct Tile<2, TK> { static constexpr int X = tile_small(TK) ? 8 : 16, Y = X, Z = 1; };
 template <> struct Tile<3, 8> { static constexpr int X = 8, Y = 8, Z = 4; };
 template <> struct Tile<3, 4> { static constexpr int X = 16, Y = 4, Z = 4; };
+template <> struct Tile<3, 8 + SMALL_TILE> { static constexpr int X = 4, Y = 4, Z = 4; };
+template <> struct Tile<3, 4 + SMALL_TILE> { static constexpr int X = 4, Y = 4, Z = 4; };
+// Cells and threads of a block, and threads that share one axis pass.
+template <int TK> constexpr int tile_cells() { return tile_small(TK) ? 64 : 256; }
+template <int D, int TK> constexpr int tile_threads() { return tile_small(TK) ? 128 * D : 256; }
+template <int TK> constexpr int pass_threads() { return tile_small(TK) ? 128 : 256; }
 
-template <int D, int A, int ES> struct TileAxis {
-  static constexpr int T = (A == 0) ? Tile<D, ES>::X : (A == 1) ? Tile<D, ES>::Y : Tile<D, ES>::Z;
-  static constexpr int LINES = 256 / T;
+template <int D, int A, int TK> struct TileAxis {
+  static constexpr int T = (A == 0) ? Tile<D, TK>::X : (A == 1) ? Tile<D, TK>::Y : Tile<D, TK>::Z;
+  static constexpr int LINES = tile_cells<TK>() / T;
   static constexpr int NSLOPE = (T + 3) * LINES;
   static constexpr int NFACE = (T + 1) * LINES;
 };
@@ -73,23 +90,30 @@ template <int MODEL, int N, int D> struct Sizes {
   static constexpr int NS = PV + D;
   // flux: alpha, mass, energ per phase (Euler: mass), momentum (D), energy, sM, uStar
   static constexpr int NF = ((MODEL == M_EULER) ? 1 : 3 * N) + D + 1 + 2;
-  // Elements staged per line of axis A (tiles of element size ES).
-  template <int A, int ES> static constexpr int per_line(bool o2) {
-    return (o2 ? (TileAxis<D, A, ES>::T + 3) * NS : 0) + (TileAxis<D, A, ES>::T + 1) * NF;
+  // Elements staged per line of axis A.
+  template <int A, int TK> static constexpr int per_line(bool o2) {
+    return (o2 ? (TileAxis<D, A, TK>::T + 3) * NS : 0) + (TileAxis<D, A, TK>::T + 1) * NF;
   }
-  // Batches of lines of axis A.
-  template <int A, int ES> static constexpr int batches(bool o2) {
+  // Batches of lines of axis A (the small tiles stage every axis whole).
+  template <int A, int TK> static constexpr int batches(bool o2) {
+    constexpr int ES = tile_esize(TK);
     int nb = 1;
-    while (nb < TileAxis<D, A, ES>::LINES && per_line<A, ES>(o2) * (TileAxis<D, A, ES>::LINES / nb) * ES > lds_batch_bytes<MODEL, ES>())
+    while (!tile_small(TK) && nb < TileAxis<D, A, TK>::LINES &&
+           per_line<A, TK>(o2) * (TileAxis<D, A, TK>::LINES / nb) * ES > lds_batch_bytes<MODEL, ES>())
       nb *= 2;
     return nb;
   }
-  template <int A, int ES> static constexpr int lds_axis(bool o2) {
-    return per_line<A, ES>(o2) * (TileAxis<D, A, ES>::LINES / batches<A, ES>(o2));
+  template <int A, int TK> static constexpr int lds_axis(bool o2) {
+    return per_line<A, TK>(o2) * (TileAxis<D, A, TK>::LINES / batches<A, TK>(o2));
   }
   static constexpr int cmax(int a, int b) { return a > b ? a : b; }
-  template <int ES> static constexpr int lds_elems(bool o2) {
-    return cmax(lds_axis<0, ES>(o2), cmax(D >= 2 ? lds_axis<1, ES>(o2) : 0, D >= 3 ? lds_axis<2, ES>(o2) : 0));
+  template <int TK> static constexpr int lds_elems(bool o2) {
+    const int a0 = lds_axis<0, TK>(o2), a1 = D >= 2 ? lds_axis<1, TK>(o2) : 0, a2 = D >= 3 ? lds_axis<2, TK>(o2) : 0;
+    return tile_small(TK) ? a0 + a1 + a2 : cmax(a0, cmax(a1, a2));
+  }
+  // Where axis A's staging starts.
+  template <int A, int TK> static constexpr int lds_base(bool o2) {
+    return !tile_small(TK) || A == 0 ? 0 : lds_axis<0, TK>(o2) + (A == 2 ? lds_axis<1, TK>(o2) : 0);
   }
 };
 
@@ -367,10 +391,11 @@ __device__ __forceinline__ void flux_from_lds(const R* o, Flux<N, R>& F) {
 // Tile origin of the block among the launch's tile rows (row0, nrows of the
 // outermost axis), XCD-aware: when the launch's tile count divides by the 8
 // XCDs, each XCD receives a contiguous range of tiles (neighbours share an L2).
-template <int D, int ES>
+template <int D, int TK>
 __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows, int& i0, int& j0, int& k0) {
-  const int t0 = (D == 1) ? nrows : P.tiles[0];
-  const int t1 = (D == 2) ? nrows : (D == 3) ? P.tiles[1] : 1;
+  const int tiles1 = tile_small(TK) ? (P.ny + Tile<D, TK>::Y - 1) / Tile<D, TK>::Y : P.tiles[1];
+  const int t0 = (D == 1) ? nrows : tile_small(TK) ? (P.nx + Tile<D, TK>::X - 1) / Tile<D, TK>::X : P.tiles[0];
+  const int t1 = (D == 2) ? nrows : (D == 3) ? tiles1 : 1;
   const int nb = t0 * t1 * ((D == 3) ? nrows : 1);
   int b = blockIdx.x;
   if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
@@ -378,7 +403,7 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
   const int rest = b / t0;
   int ty = rest % t1;
   int tz = rest / t1;
-  if (D == 3 && ES == 4 && (t1 & 1) == 0 && (nrows & 1) == 0) {
+  if (D == 3 && TK == 4 && (t1 & 1) == 0 && (nrows & 1) == 0) {
     // 3D FP32 tiles (16 x 4 x 4): rows of x tiles in 2 x 2 groups over (y, z), so
     // that the y and the z neighbours of a row run close in time and meet their
     // shared halo planes in L2 (the 512^3 step fetches 13 % less).
@@ -389,26 +414,27 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
   if (D == 1) tx += row0;
   else if (D == 2) ty += row0;
   else tz += row0;
-  i0 = tx * Tile<D, ES>::X;
-  j0 = ty * Tile<D, ES>::Y;
-  k0 = tz * Tile<D, ES>::Z;
+  i0 = tx * Tile<D, TK>::X;
+  j0 = ty * Tile<D, TK>::Y;
+  k0 = tz * Tile<D, TK>::Z;
 }
 
 // One axis pass (steps A, B, C above) for axis AX with face frame FR, in
-// batches of lines when the staging would exceed lds_batch_bytes.
-template <int MODEL, int N, int D, bool O2, typename R, int LK, int AX, int FR>
+// batches of lines when the staging would exceed lds_batch_bytes.  The small tiles call
+// one step at a time (STEPS) on the axis's own threads, with the barriers between them.
+constexpr int STEP_A = 1, STEP_B = 2, STEP_C = 4, STEP_ABC = 7;
+template <int MODEL, int N, int D, bool O2, typename R, int LK, int AX, int FR, int TK = (int)sizeof(R), int STEPS = STEP_ABC>
 __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>& L, R* lds, const int org[3],
                                           const int own[3], bool own_ok, const R* an, const R* pn, R& smax,
                                           ConsAcc<N, R>& acc) {
-  constexpr int ES = (int)sizeof(R);
-  using TA = TileAxis<D, AX, ES>;
+  using TA = TileAxis<D, AX, TK>;
   using SZ = Sizes<MODEL, N, D>;
   constexpr int T = TA::T;
-  constexpr int NB = SZ::template batches<AX, ES>(O2);
+  constexpr int NB = SZ::template batches<AX, TK>(O2);
   constexpr int LB = TA::LINES / NB;              // lines per batch
   constexpr int B = (AX == 0) ? 1 : 0;           // first line axis
   constexpr int C = (AX == 2) ? 1 : 2;           // second line axis
-  constexpr int TB = (B == 0) ? Tile<D, ES>::X : Tile<D, ES>::Y;
+  constexpr int TB = (B == 0) ? Tile<D, TK>::X : Tile<D, TK>::Y;
   // Cell indices: 32-bit from the launch's first cell in FP32, 64-bit in FP64.
   using CI = typename std::conditional<off32<R>(), uint32_t, int64_t>::type;
   const int n3[3] = {P.nx, P.ny, P.nz};
@@ -416,8 +442,8 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
   const CI cb0 = off32<R>() ? (CI)L.cbase : CI(0);
   const int na = n3[AX];
   const CI sa = st3[AX];
-  R* s_slope = lds;
-  R* s_flux = lds + (O2 ? (T + 3) * LB * SZ::NS : 0);
+  R* s_slope = lds + SZ::template lds_base<AX, TK>(O2);
+  R* s_flux = s_slope + (O2 ? (T + 3) * LB * SZ::NS : 0);
   // Face slopes: slot g of line lb is s = lb * (T + 3) + g + 2.  A slope of NS
   // elements whose bytes are a multiple of 32 (8 doubles in 2D with two phases,
   // 12 in 3D with three; 8 floats in 2D) is staged variable-major, element v at
@@ -436,7 +462,7 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
   constexpr int NREC = (T + 1) * LB;
   constexpr int FRS = (sizeof(R) == 8) ? 1 : SZ::NF;     // record stride
   constexpr int FES = (sizeof(R) == 8) ? NREC : 1;       // element stride
-  const int tid = threadIdx.x;
+  const int tid = tile_small(TK) ? threadIdx.x % pass_threads<TK>() : threadIdx.x;
   const int lown = (own[B] - org[B]) + TB * (own[C] - org[C]);   // line of the own cell
   // Work slots of steps A and B run along the axis for x (contiguous cells), and
   // across the lines for y and z, whose consecutive lines are consecutive x: a
@@ -450,8 +476,8 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
   for (int bt = 0; bt < NB; bt++) {
     const int l0 = bt * LB;
     // A. face slopes s_g, g = -2 .. T (interior faces only)
-    if (O2) {
-      for (int q = tid; q < (T + 3) * LB; q += 256) {
+    if constexpr (O2 && (STEPS & STEP_A)) {
+      for (int q = tid; q < (T + 3) * LB; q += pass_threads<TK>()) {
         const int g = (ACROSS ? q / LB : q % (T + 3)) - 2;
         const int lb = ACROSS ? q % LB : q / (T + 3);
         const int l = l0 + lb;
@@ -472,62 +498,64 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
           wall_slope_vars<MODEL, N, D, R, SES>(cw, AX, m < 0 ? pv<R>(P.dwall[AX][0], P.f_dwall[AX][0]) : -pv<R>(P.dwall[AX][1], P.f_dwall[AX][1]), o);
         }
       }
-      __syncthreads();
+      if (STEPS == STEP_ABC) __syncthreads();
     }
 
     // B. interior face fluxes f = -1 .. T-1
-    for (int q = tid; q < (T + 1) * LB; q += 256) {
-      const int f = (ACROSS ? q / LB : q % (T + 1)) - 1;
-      const int lb = ACROSS ? q % LB : q / (T + 1);
-      const int l = l0 + lb;
-      const int cb = org[B] + l % TB, cc = org[C] + l / TB;
-      const int m = org[AX] + f;
-      if (cb < n3[B] && cc < n3[C] && m >= 0 && m <= na - 2) {
-        const CI cell = (CI)m * sa + (CI)cb * st3[B] + (CI)cc * st3[C] - cb0;
-        Cell<N, R> bl, br;
-        load_prim<MODEL, N, D, off32<R>()>(P, L.wsrc, cell, bl);
-        load_prim<MODEL, N, D, off32<R>()>(P, L.wsrc, cell + sa, br);
-        if (O2) {
-          const R aL = (MODEL == M_EULER) ? R(0.) : bl.a[0];
-          const R aR = (MODEL == M_EULER) ? R(0.) : br.a[0];
-          const R* s1 = s_slope + (lb * (T + 3) + f + 2) * SRS;
-          const bool hasm = (m >= 1) || wall_m, hasp = (m + 1 <= na - 2) || wall_p;
-          // The far neighbours' time-n alpha only decides the interface limiter switch;
-          // across a wall the "cell after" is the cell itself (CellO2Cartesian.cpp:75-79).
-          const R aLL = (LK < 0 && MODEL != M_EULER && hasm) ? alpha0_at<R>(L.wn, (m >= 1) ? cell - sa : cell) : R(0.);
-          const R aRR = (LK < 0 && MODEL != M_EULER && hasp)
-                            ? alpha0_at<R>(L.wn, (m + 1 <= na - 2) ? cell + 2 * sa : cell + sa)
-                            : R(0.);
-          extrapolate<MODEL, N, D, R, LK, SES>(P, bl, s1, s1 - SRS, hasm, aLL, aL, aR, face_dfl<R, AX>(P, m), false);
-          extrapolate<MODEL, N, D, R, LK, SES>(P, br, s1, s1 + SRS, hasp, aRR, aR, aL, face_dfr<R, AX>(P, m), true);
-          if constexpr (LK == LK_FULL && MODEL != M_EULER && N == 2) {
-            if (P.thinc) {
-              // THINC replaces the extrapolated volume fractions at an interface.
-              double na;
-              if (thinc_alpha(P, 0, (double)aL, (double)aLL, (double)aR, na)) { bl.a[0] = R(na); bl.a[1] = R(1. - na); }
-              if (thinc_alpha(P, 1, (double)aR, (double)aRR, (double)aL, na)) { br.a[0] = R(na); br.a[1] = R(1. - na); }
+    if constexpr (STEPS & STEP_B) {
+      for (int q = tid; q < (T + 1) * LB; q += pass_threads<TK>()) {
+        const int f = (ACROSS ? q / LB : q % (T + 1)) - 1;
+        const int lb = ACROSS ? q % LB : q / (T + 1);
+        const int l = l0 + lb;
+        const int cb = org[B] + l % TB, cc = org[C] + l / TB;
+        const int m = org[AX] + f;
+        if (cb < n3[B] && cc < n3[C] && m >= 0 && m <= na - 2) {
+          const CI cell = (CI)m * sa + (CI)cb * st3[B] + (CI)cc * st3[C] - cb0;
+          Cell<N, R> bl, br;
+          load_prim<MODEL, N, D, off32<R>()>(P, L.wsrc, cell, bl);
+          load_prim<MODEL, N, D, off32<R>()>(P, L.wsrc, cell + sa, br);
+          if (O2) {
+            const R aL = (MODEL == M_EULER) ? R(0.) : bl.a[0];
+            const R aR = (MODEL == M_EULER) ? R(0.) : br.a[0];
+            const R* s1 = s_slope + (lb * (T + 3) + f + 2) * SRS;
+            const bool hasm = (m >= 1) || wall_m, hasp = (m + 1 <= na - 2) || wall_p;
+            // The far neighbours' time-n alpha only decides the interface limiter switch;
+            // across a wall the "cell after" is the cell itself (CellO2Cartesian.cpp:75-79).
+            const R aLL = (LK < 0 && MODEL != M_EULER && hasm) ? alpha0_at<R>(L.wn, (m >= 1) ? cell - sa : cell) : R(0.);
+            const R aRR = (LK < 0 && MODEL != M_EULER && hasp)
+                              ? alpha0_at<R>(L.wn, (m + 1 <= na - 2) ? cell + 2 * sa : cell + sa)
+                              : R(0.);
+            extrapolate<MODEL, N, D, R, LK, SES>(P, bl, s1, s1 - SRS, hasm, aLL, aL, aR, face_dfl<R, AX>(P, m), false);
+            extrapolate<MODEL, N, D, R, LK, SES>(P, br, s1, s1 + SRS, hasp, aRR, aR, aL, face_dfr<R, AX>(P, m), true);
+            if constexpr (LK == LK_FULL && MODEL != M_EULER && N == 2) {
+              if (P.thinc) {
+                // THINC replaces the extrapolated volume fractions at an interface.
+                double na;
+                if (thinc_alpha(P, 0, (double)aL, (double)aLL, (double)aR, na)) { bl.a[0] = R(na); bl.a[1] = R(1. - na); }
+                if (thinc_alpha(P, 1, (double)aR, (double)aRR, (double)aL, na)) { br.a[0] = R(na); br.a[1] = R(1. - na); }
+              }
             }
+            derive<MODEL, N, R>(P, bl, MODEL == M_EULER);
+            derive<MODEL, N, R>(P, br, MODEL == M_EULER);
+          } else {
+            derive<MODEL, N, R>(P, bl, false);
+            derive<MODEL, N, R>(P, br, false);
           }
-          derive<MODEL, N, R>(P, bl, MODEL == M_EULER);
-          derive<MODEL, N, R>(P, br, MODEL == M_EULER);
-        } else {
-          derive<MODEL, N, R>(P, bl, false);
-          derive<MODEL, N, R>(P, br, false);
+          Flux<N, R> F;
+          face_flux<MODEL, N, FR, R, crpow<R, LK>()>(P, bl, bl.E, br, br.E, smax, F);
+          flux_to_lds<MODEL, N, D, FES, R>(F, s_flux + (lb * (T + 1) + f + 1) * FRS);
+        } else if (sizeof(R) == 4 && cb < n3[B] && cc < n3[C]) {
+          // The FP32 gather reads both faces of every cell: a face outside the mesh is zero.
+          R* o = s_flux + (lb * (T + 1) + f + 1) * SZ::NF;
+  #pragma unroll
+          for (int v = 0; v < SZ::NF; v++) o[v] = R(0.);
         }
-        Flux<N, R> F;
-        face_flux<MODEL, N, FR, R, crpow<R, LK>()>(P, bl, bl.E, br, br.E, smax, F);
-        flux_to_lds<MODEL, N, D, FES, R>(F, s_flux + (lb * (T + 1) + f + 1) * FRS);
-      } else if (sizeof(R) == 4 && cb < n3[B] && cc < n3[C]) {
-        // The FP32 gather reads both faces of every cell: a face outside the mesh is zero.
-        R* o = s_flux + (lb * (T + 1) + f + 1) * SZ::NF;
-#pragma unroll
-        for (int v = 0; v < SZ::NF; v++) o[v] = R(0.);
       }
     }
-    __syncthreads();
+    if (STEPS == STEP_ABC) __syncthreads();
 
     // C. gather: add the lower face, subtract the upper face
-    if (own_ok && lown / LB == bt) {
+    if ((STEPS & STEP_C) && own_ok && lown / LB == bt) {
       const int t = own[AX] - org[AX];
       const int lb = lown - l0;
       const R coef = pv<R>(P.coef[AX], P.f_coef[AX]);
@@ -548,7 +576,7 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
         }
       }
     }
-    __syncthreads();
+    if (STEPS == STEP_ABC) __syncthreads();
   }
 }
 
@@ -751,7 +779,7 @@ __device__ __forceinline__ void capture_samples(const SampleSink& K, bool cap, c
 // LDS of one wave in the learned kernels after the flux passes: the inference's
 // staging (MLP_WAVE_LDS) and two doubles per lane for the start's affine form.
 constexpr int STEP_WAVE_LDS = MLP_WAVE_LDS + 64 * 2 * 8;
-constexpr int STEP_BLOCK_LDS = 4 * STEP_WAVE_LDS;
+template <int TK> constexpr int step_block_lds() { return tile_cells<TK>() / 64 * STEP_WAVE_LDS; }   // waves with cells
 
 template <typename R, int N, int D, bool O2, bool LEARN, int LK>
 constexpr int step_waves() {
@@ -762,26 +790,26 @@ constexpr int step_waves() {
 // relaxing kernels with a sample buffer attached; the full-featured kernels
 // always carry it).  Without it the capture path is not compiled: its features
 // and slot arithmetic cost the FP64 benchmark kernel 1 % even when not taken.
-template <int MODEL, int N, int D, bool O2, typename R, bool LEARN, int LK, bool CAP = false>
-__global__ __launch_bounds__(256, (step_waves<R, N, D, O2, LEARN, LK>())) void k_step(ParamsPtr Pc, StepLaunchT<R> L, Clock* __restrict__ clk,
+template <int MODEL, int N, int D, bool O2, typename R, bool LEARN, int LK, bool CAP = false, int TK = (int)sizeof(R)>
+__global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, LEARN, LK>())) void k_step(ParamsPtr Pc, StepLaunchT<R> L, Clock* __restrict__ clk,
                                               Counters* __restrict__ cnt) {
   constexpr bool CAPTURE = !LEARN && MODEL != M_EULER && (CAP || LK == LK_FULL);
   const Params& P = *(const Params*)Pc;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   R* lds = reinterpret_cast<R*>(lds_raw);
-  __shared__ double s_dt[4], s_res[4];
-  __shared__ unsigned long long s_c[6][4];
+  constexpr int NW = tile_threads<D, TK>() / 64;   // waves of the block
+  __shared__ double s_dt[NW], s_res[NW];
+  __shared__ unsigned long long s_c[6][NW];
   if (clk->done) return;
   const double dt = clk->dt;
   int org[3];
-  constexpr int ES = (int)sizeof(R);
-  tile_origin<D, ES>(P, L.row0, L.nrows, org[0], org[1], org[2]);
+  tile_origin<D, TK>(P, L.row0, L.nrows, org[0], org[1], org[2]);
   const int tid = threadIdx.x;
   int own[3];
-  own[0] = org[0] + tid % Tile<D, ES>::X;
-  own[1] = org[1] + (tid / Tile<D, ES>::X) % Tile<D, ES>::Y;
-  own[2] = org[2] + tid / (Tile<D, ES>::X * Tile<D, ES>::Y);
-  const bool own_ok = own[0] < P.nx && own[1] < P.ny && own[2] < P.nz;
+  own[0] = org[0] + tid % Tile<D, TK>::X;
+  own[1] = org[1] + (tid / Tile<D, TK>::X) % Tile<D, TK>::Y;
+  own[2] = org[2] + tid / (Tile<D, TK>::X * Tile<D, TK>::Y);
+  const bool own_ok = (!tile_small(TK) || tid < tile_cells<TK>()) && own[0] < P.nx && own[1] < P.ny && own[2] < P.nz;
   const int64_t c = own[0] + (int64_t)own[1] * P.nx + (int64_t)own[2] * P.nx * P.ny;
   const int64_t lc = c - (off32<R>() ? (int64_t)L.cbase : 0);   // state index of the own cell
 
@@ -801,9 +829,28 @@ __global__ __launch_bounds__(256, (step_waves<R, N, D, O2, LEARN, LK>())) void k
   }
   ConsAcc<N, R> acc;
 
-  axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
-  if (D >= 2) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
-  if (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+  if constexpr (tile_small(TK)) {
+    // Waves 0-1 take the x axis, 2-3 y, 4-5 z; the first wave gathers in the faces' order.
+    const int grp = __builtin_amdgcn_readfirstlane(tid / pass_threads<TK>());
+#define ECG_AXES(STEP)                                                                                               \
+  do {                                                                                                               \
+    if (grp == 0) axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
+    else if (grp == 1) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
+    else if constexpr (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
+    __syncthreads();                                                                                                 \
+  } while (0)
+    if constexpr (O2) ECG_AXES(STEP_A);
+    ECG_AXES(STEP_B);
+#undef ECG_AXES
+    axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    if constexpr (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    __syncthreads();
+  } else {
+    axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    if (D >= 2) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    if (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+  }
 
   Cell<N> nw;
   bool relax_now = false, spread_ok = false;
@@ -1002,7 +1049,7 @@ __global__ __launch_bounds__(256, (step_waves<R, N, D, O2, LEARN, LK>())) void k
   if (threadIdx.x == 0) {
     double m = s_dt[0], rs = s_res[0];
     unsigned long long a = s_c[0][0], b = s_c[1][0], r = s_c[2][0], w = s_c[3][0], wf = s_c[4][0], nb = s_c[5][0];
-    for (int q = 1; q < 4; q++) {
+    for (int q = 1; q < NW; q++) {
       m = dmax<double>(m, s_dt[q]); rs += s_res[q];
       a += s_c[0][q]; b += s_c[1][q]; r += s_c[2][q]; w += s_c[3][q]; wf += s_c[4][q]; nb += s_c[5][q];
     }
@@ -1088,18 +1135,43 @@ __global__ __launch_bounds__(256) void k_fill(Params P, const DomainDev* __restr
   store_prim<MODEL, N, D>(P, W, c, s);
 }
 
+// The small tiles serve meshes whose ordinary tiles leave most of the chip's 256 CUs
+// empty, where a stage lasts as long as one block: up to 256 ordinary tiles at second order
+// in 2D and in FP32, up to 128 at first order and in 3D FP64, where a block's chain is
+// shorter against the small tiles' extra faces.  Both sides measured, a step on caller
+// buffers, ordinary / small tiles (us): 2D two-phase O2 FP64 96^2 90/63, 256^2 87/86, 304^2
+// 93/95, FP32 256^2 71/63; 3D two-phase O2 FP32 32^3 79/63, 44^3 91/107; 2D O1 FP64 160^2
+// 50/46, 256^2 52/55; 3D two-phase O2 FP64 24^3 109/67, 32^3 103/91, 40^3 111/137; Euler
+// O2 FP64 32^3 69/53, 48^3 78/91.  The full-featured and the capture kernels keep the
+// ordinary tiles (their code is long; Euler's LK_FULL, the second-order walls, is the
+// exception).
+template <int MODEL, int D, int LK, bool CAP> constexpr bool has_small() {
+  return D >= 2 && !CAP && (LK != LK_FULL || MODEL == M_EULER);
+}
+template <int D, bool O2, int ES> inline bool step_small(const Params& P) {
+  return (int64_t)P.tiles[0] * P.tiles[1] * P.tiles[2] <= ((O2 && (D == 2 || ES == 4)) ? 256 : 128);
+}
+
 // One stage of the step.  The FP32 kernels address the state by 32-bit byte
 // offsets from the launch's first cell: when the tile rows of the outermost axis
 // (with the two lines of halo on each side) span more than step_span_bytes of
 // one variable, the stage runs as several launches over consecutive rows (an
 // even count each, for the FP32 tile groups), each with its own first cell.
-template <int MODEL, int N, int D, bool O2, typename R, bool LEARN, int LK, bool CAP = false>
+template <int MODEL, int N, int D, bool O2, typename R, bool LEARN, int LK, bool CAP = false, int TK = (int)sizeof(R)>
 void launch_step_v(const Params& P, const StepLaunchT<R>& L, Clock* clk, Counters* cnt, hipStream_t s) {
-  using SZ = Sizes<MODEL, N, D>;
   constexpr int ES = (int)sizeof(R);
-  constexpr int T = (D == 3) ? Tile<D, ES>::Z : (D == 2) ? Tile<D, ES>::Y : Tile<D, ES>::X;
-  const int rows = P.tiles[D - 1];
-  const int per_row = P.tiles[0] * P.tiles[1] * P.tiles[2] / rows;   // blocks of one tile row
+  if constexpr (!tile_small(TK) && has_small<MODEL, D, LK, CAP>()) {
+    if (step_small<D, O2, ES>(P)) {
+      launch_step_v<MODEL, N, D, O2, R, LEARN, LK, CAP, TK + SMALL_TILE>(P, L, clk, cnt, s);
+      return;
+    }
+  }
+  using SZ = Sizes<MODEL, N, D>;
+  using TL = Tile<D, TK>;
+  constexpr int T = (D == 3) ? TL::Z : (D == 2) ? TL::Y : TL::X;
+  const int t3[3] = {(P.nx + TL::X - 1) / TL::X, (P.ny + TL::Y - 1) / TL::Y, (P.nz + TL::Z - 1) / TL::Z};
+  const int rows = t3[D - 1];
+  const int per_row = t3[0] * t3[1] * t3[2] / rows;   // blocks of one tile row
   const int64_t line = (D == 3) ? (int64_t)P.nx * P.ny : (D == 2) ? (int64_t)P.nx : 1;   // cells of one line
   int chunk = rows;
   if (off32<R>()) {
@@ -1107,9 +1179,9 @@ void launch_step_v(const Params& P, const StepLaunchT<R>& L, Clock* clk, Counter
     chunk = (int)std::min<int64_t>(rows, std::max<int64_t>((lines - 4) / T, 1));
     if (chunk < rows && chunk > 1) chunk &= ~1;
   }
-  size_t lds = sizeof(R) * SZ::template lds_elems<ES>(O2);
-  if (LEARN && lds < (size_t)STEP_BLOCK_LDS) lds = STEP_BLOCK_LDS;
-  auto k = k_step<MODEL, N, D, O2, R, LEARN, LK, CAP>;
+  size_t lds = sizeof(R) * SZ::template lds_elems<TK>(O2);
+  if (LEARN && lds < (size_t)step_block_lds<TK>()) lds = step_block_lds<TK>();
+  auto k = k_step<MODEL, N, D, O2, R, LEARN, LK, CAP, TK>;
   // A failure here surfaces as the launch error the caller checks next.
   (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   for (int r0 = 0; r0 < rows; r0 += chunk) {
@@ -1124,7 +1196,7 @@ void launch_step_v(const Params& P, const StepLaunchT<R>& L, Clock* clk, Counter
       Ls.wsrc = L.wsrc + first;
       Ls.wout = L.wout + first;
     }
-    hipLaunchKernelGGL(k, dim3(per_row * Ls.nrows), dim3(256), lds, s, (ParamsPtr)L.pdev, Ls, clk, cnt);
+    hipLaunchKernelGGL(k, dim3(per_row * Ls.nrows), dim3(tile_threads<D, TK>()), lds, s, (ParamsPtr)L.pdev, Ls, clk, cnt);
   }
 }
 
