@@ -647,19 +647,34 @@ __device__ __forceinline__ double wave_min(double v) {
   for (int o = 32; o > 0; o >>= 1) v = dmin<double>(v, __shfl_xor(v, o, 64));
   return v;
 }
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = dmax<double>(v, __shfl_xor(v, o, 64));
-  return v;
-}
 __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+
+// The step kernels' wave reductions, by DPP moves (row shifts, then the row broadcasts of a
+// 64-wide wave; lane 63 ends with the whole): no LDS pipe, and a few cycles a step where a
+// cross-lane permute is a round trip of about a hundred.  Lanes without a source take 0, the
+// identity of both reductions (speeds are not negative).
+template <int CTRL, int ROWS> __device__ __forceinline__ uint32_t dpp0(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ float dpp0(float x) {
+  return __builtin_bit_cast(float, dpp0<CTRL, ROWS>(__builtin_bit_cast(uint32_t, x)));
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp0(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  return __builtin_bit_cast(double, (uint64_t)dpp0<CTRL, ROWS>((uint32_t)b) |
+                                        ((uint64_t)dpp0<CTRL, ROWS>((uint32_t)(b >> 32)) << 32));
+}
+template <typename T, class Op> __device__ __forceinline__ T wave_reduce63(T v, Op op) {
+  v = op(v, dpp0<0x111, 0xf>(v));   // row_shr 1, 2, 4, 8
+  v = op(v, dpp0<0x112, 0xf>(v));
+  v = op(v, dpp0<0x114, 0xf>(v));
+  v = op(v, dpp0<0x118, 0xf>(v));
+  v = op(v, dpp0<0x142, 0xa>(v));   // row_bcast 15 into rows 1 and 3
+  v = op(v, dpp0<0x143, 0xc>(v));   // row_bcast 31 into rows 2 and 3
   return v;
 }
 
@@ -1028,31 +1043,44 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
     n_bad = nonfinite_prim<MODEL, N, D>(nw) ? 1 : 0;
     store_prim<MODEL, N, D, off32<R>()>(P, L.wout, lc, nw);
   }
-  // Block reductions: largest wave speed (the CFL bound) and relaxation counters.
-  // The counters take one wave sum, packed in bit fields wide enough for a wave:
-  // evaluations (at most 64 x 200) in 16 bits, each per-cell flag in 8.
-  const double smax64 = wave_max((double)smax);
-  const unsigned long long ps = wave_sum(n_it | (n_relax << 16) | (n_warm << 24) | (n_wfb << 32) | (n_fail << 40) |
-                                         (n_warn << 48) | (n_bad << 56));
-  resid = wave_sum_d(resid);
+  // Block reductions: largest wave speed (the CFL bound) and relaxation counters (per-cell
+  // flags by ballot).
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    s_dt[wv] = smax64; s_res[wv] = resid;
-    s_c[0][wv] = ps & 0xFFFFull;
-    s_c[1][wv] = ((ps >> 40) & 0xFFull) | (((ps >> 48) & 0xFFull) << 32);   // failures, warnings in the high half
-    s_c[2][wv] = (ps >> 16) & 0xFFull;
-    s_c[3][wv] = (ps >> 24) & 0xFFull;
-    s_c[4][wv] = (ps >> 32) & 0xFFull;
-    s_c[5][wv] = ps >> 56;
+  const R wmax = wave_reduce63(smax, [](R a, R b) { return dmax<R>(a, b); });
+  const unsigned nb_w = __popcll(__ballot(n_bad != 0));
+  unsigned nr_w = 0, it_w = 0, nw_w = 0, nf_w = 0, fail_w = 0, warn_w = 0;
+  if constexpr (MODEL != M_EULER) {
+    nr_w = __popcll(__ballot(n_relax != 0));
+    if (nr_w) {
+      it_w = wave_reduce63((uint32_t)n_it, [](uint32_t a, uint32_t b) { return a + b; });
+      resid = wave_reduce63(resid, [](double a, double b) { return a + b; });
+      fail_w = __popcll(__ballot(n_fail != 0));
+      warn_w = __popcll(__ballot(n_warn != 0));
+      if constexpr (LEARN) {
+        nw_w = __popcll(__ballot(n_warm != 0));
+        nf_w = __popcll(__ballot(n_wfb != 0));
+      }
+    }
+  }
+  if (lane == 63) {
+    s_dt[wv] = (double)wmax;
+    s_c[5][wv] = nb_w;
+    if constexpr (MODEL != M_EULER) {
+      s_res[wv] = resid;
+      s_c[0][wv] = it_w; s_c[1][wv] = fail_w | ((unsigned long long)warn_w << 32);   // warnings in the high half
+      s_c[2][wv] = nr_w; s_c[3][wv] = nw_w; s_c[4][wv] = nf_w;
+    }
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double m = s_dt[0], rs = s_res[0];
-    unsigned long long a = s_c[0][0], b = s_c[1][0], r = s_c[2][0], w = s_c[3][0], wf = s_c[4][0], nb = s_c[5][0];
-    for (int q = 1; q < NW; q++) {
-      m = dmax<double>(m, s_dt[q]); rs += s_res[q];
-      a += s_c[0][q]; b += s_c[1][q]; r += s_c[2][q]; w += s_c[3][q]; wf += s_c[4][q]; nb += s_c[5][q];
-    }
+    double m = s_dt[0], rs = 0.;
+    unsigned long long a = 0, b = 0, r = 0, w = 0, wf = 0, nb = s_c[5][0];
+    for (int q = 1; q < NW; q++) { m = dmax<double>(m, s_dt[q]); nb += s_c[5][q]; }
+    if constexpr (MODEL != M_EULER)
+      for (int q = 0; q < NW; q++) {
+        rs += s_res[q];
+        a += s_c[0][q]; b += s_c[1][q]; r += s_c[2][q]; w += s_c[3][q]; wf += s_c[4][q];
+      }
     Counters* slot = cnt + (blockIdx.x % ATOMIC_SLOTS);
     const double dtb = cfl_dt(P.lcfl, m);
     atomicMin(&slot->dtmax_bits, (unsigned long long)__double_as_longlong(dtb));
