@@ -217,7 +217,6 @@ struct ecg_ctx {
   void* W[3] = {nullptr, nullptr, nullptr};    // two time levels + second-order predicted state
   int esize = 8;                               // bytes per state element (8: FP64 form, 4: FP32 forms)
   int cur = 0;                                 // W[cur] holds the current state
-  double* tables = nullptr;
   double* tank_buf = nullptr;                  // flux records of the inlet-tank faces (k_tank)
   int64_t ntank = 0;                           // inlet-tank faces
   Params* pdev = nullptr;                      // device copy of P (the step kernels' parameters)
@@ -426,26 +425,15 @@ static int check_config(const ecg_config* c) {
   return ECG_OK;
 }
 
-// The three distances of interior face m of an axis with cell size d, cells m | m + 1
-// (Element.cpp:77-81, Face.cpp:52-56): which = 0 centre to centre, 1 face to the left
-// centre, 2 face to the right centre.  Centres at (i + 0.5) d (MeshCartesian.cpp:178).
-__host__ __device__ inline double face_distance(double d, int m, int which) {
-  const double pm = (m + 0.5) * d, pp = (m + 1 + 0.5) * d;
-  const double fp = pm + 0.5 * d;
-  const double x = (which == 0) ? pm - pp : (which == 1) ? fp - pm : fp - pp;
-  return sqrt(x * x + 0. * 0. + 0. * 0.);
-}
-
-// Sizes of a case's state and tables.
+// Sizes of a case's state.
 struct Layout {
   int D, nvar, esize;
   int64_t ncell, pitch, ntank;
-  size_t tab_off[3][3], ntab;   // distance tables: offsets (doubles) of axis a, kind k; total
 };
 
 // Everything the step kernels' parameters hold that needs no device memory: geometry,
 // EOS, limiters, boundaries, tanks, tiles and the uniform-axis constants.  The device
-// pointers (tables, tank records, warning log) are the caller's to set.  Allocates
+// pointers (tank records, warning log) are the caller's to set.  Allocates
 // nothing.  g is a checked configuration with relax_p normalised.
 static void build_params(const ecg_config& g, Params& P, Layout& Ly) {
   Ly.D = (g.nx > 1) + (g.ny > 1) + (g.nz > 1);
@@ -472,6 +460,14 @@ static void build_params(const ecg_config& g, Params& P, Layout& Ly) {
   if (Ly.D > 1) lcfl *= 0.6;
   P.lcfl = lcfl;
   P.eps = (g.model != ECG_EULER && g.alpha_null) ? 1.e-15 : 0.;  // Eos.cpp:88-97
+  // verifyAndCorrectPhase (PhaseUEq.cpp:355-370), in each arithmetic.
+  CellFloors& q = P.floors;
+  const bool an = P.eps > 1.e-20;
+  q.alo = an ? 0. : 1e-15;       q.f_alo = an ? 0.f : (float)1e-15;
+  q.alo_v = an ? 0. : 1e-14;     q.f_alo_v = an ? 0.f : (float)1e-14;
+  q.ahi = an ? 1. : 1. - 1e-15;  q.f_ahi = an ? 1.f : 1.f - (float)1e-15;
+  q.ahi_v = an ? 1. : 1. - 1e-14; q.f_ahi_v = an ? 1.f : 1.f - (float)1e-14;
+  q.rho_v = an ? 1.e-15 : 1.e-14; q.f_rho_v = an ? (float)1.e-15 : (float)1.e-14;
   P.cfl = g.cfl;
   P.alpha_null = g.alpha_null;
   P.relax = g.relax_p;
@@ -498,14 +494,10 @@ static void build_params(const ecg_config& g, Params& P, Layout& Ly) {
     P.dwall[a][0] = std::sqrt(x0 * x0 + 0. * 0. + 0. * 0.);
     P.dwall[a][1] = std::sqrt(x1 * x1 + 0. * 0. + 0. * 0.);
   }
-  // Distance tables of the interior faces: their layout, and the axes where each of the
-  // three distances is one value.
-  Ly.ntab = 0;
+  // The axes where each of the three face distances is one value.
   P.dist_uniform = 0;
   P.dcc_pow2 = 0;
   for (int a = 0; a < 3; a++) {
-    const size_t nf = (size_t)std::max(n3[a] - 1, 1);
-    for (int k = 0; k < 3; k++) { Ly.tab_off[a][k] = Ly.ntab; Ly.ntab += nf; }
     if (n3[a] < 2) continue;
     const double c0 = face_distance(P.d[a], 0, 0), l0 = face_distance(P.d[a], 0, 1), r0 = face_distance(P.d[a], 0, 2);
     bool uni = true;
@@ -560,11 +552,6 @@ ecg_ctx* ecg_create(const ecg_config* cfg) {
     delete c;
     return nullptr;
   }
-  const int n3[3] = {g.nx, g.ny, g.nz};
-  std::vector<double> tab(Ly.ntab, 0.);
-  for (int a = 0; a < 3; a++)
-    for (int m = 0; m + 1 < n3[a]; m++)
-      for (int k = 0; k < 3; k++) tab[Ly.tab_off[a][k] + m] = face_distance(P.d[a], m, k);
   bool ok = true;
   auto chk = [&](hipError_t e, const char* what) {
     if (e != hipSuccess && ok) {
@@ -576,8 +563,6 @@ ecg_ctx* ecg_create(const ecg_config* cfg) {
   const size_t bytes = (size_t)c->esize * (size_t)c->pitch * c->nvar;
   const int nbuf = (g.order == 2) ? 3 : 2;
   for (int b = 0; b < nbuf && ok; b++) chk(hipMalloc(&c->W[b], bytes), "hipMalloc(state)");
-  if (ok) chk(hipMalloc(&c->tables, sizeof(double) * tab.size()), "hipMalloc(tables)");
-  if (ok) chk(hipMemcpy(c->tables, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice), "hipMemcpy(tables)");
   const int64_t ntank = Ly.ntank;
   if (ok && ntank > 0) chk(hipMalloc(&c->tank_buf, sizeof(double) * TANK_REC * ntank), "hipMalloc(tank records)");
   c->ntank = ntank;
@@ -599,11 +584,6 @@ ecg_ctx* ecg_create(const ecg_config* cfg) {
   // memory can come back from an earlier context with its old contents).
   std::memset(c->hclk, 0, sizeof(Clock));
   std::memset(c->hcnt, 0, sizeof(Counters) * ATOMIC_SLOTS);
-  for (int a = 0; a < 3; a++) {
-    P.dcc[a] = c->tables + Ly.tab_off[a][0];
-    P.dfl[a] = c->tables + Ly.tab_off[a][1];
-    P.dfr[a] = c->tables + Ly.tab_off[a][2];
-  }
   // The step kernels' parameters, complete from here on.
   if (hipMalloc(&c->pdev, sizeof(Params)) != hipSuccess ||
       hipMemcpy(c->pdev, &c->P, sizeof(Params), hipMemcpyHostToDevice) != hipSuccess) {
@@ -633,7 +613,6 @@ void ecg_destroy(ecg_ctx* c) {
   if (c->warn_cnt) hipFree(c->warn_cnt);
   for (int b = 0; b < 3; b++)
     if (c->W[b]) hipFree(c->W[b]);
-  if (c->tables) hipFree(c->tables);
   if (c->tank_buf) hipFree(c->tank_buf);
   if (c->clk) hipFree(c->clk);
   if (c->cnt) hipFree(c->cnt);
@@ -1216,7 +1195,7 @@ int ecg_kernel_times(ecg_ctx* c, double* ms_total, int64_t* launches, int nkinds
 // ---------------------------------------------------------------------------
 // Everything the step needs beyond the caller's two state buffers lives in this
 // file-scope device array: the parameter copy, the clock, the counter slots, the
-// warning counter, the distance tables, the inlet-tank records and, at second order,
+// warning counter, the inlet-tank records and, at second order,
 // the predicted state W*.  Each GPU the library runs on holds its own copy until the
 // process ends.  In host code `scratch` names a host-side stand-in, not device memory:
 // the device address of each GPU's copy comes from hipGetSymbolAddress, once per device
@@ -1246,42 +1225,26 @@ static int noalloc_scratch(unsigned char** out) {
 }
 
 // Everything a step on caller buffers finds in the scratch array, in one launch: the
-// parameter copy, zeroed counter slots (dtMax slots at 1e10), the zeroed warning counter,
-// the given clock (block 0) and the distance tables of the interior faces, the same
-// arithmetic as the host's.  Bound by latency alone: as a host copy and two kernels it
-// took three dependent submissions ahead of every step.
+// parameter copy, zeroed counter slots (dtMax slots at 1e10), the zeroed warning counter and
+// the given clock.  Bound by latency alone: as a host copy and two kernels it took three
+// dependent submissions ahead of every step.
 __global__ __launch_bounds__(256) void k_noalloc_open(Params P, Params* pdev, Clock* clk, Counters* cnt,
-                                                      unsigned long long* warn_cnt, Clock v, double* tab, int64_t o0,
-                                                      int64_t o1, int64_t o2) {
+                                                      unsigned long long* warn_cnt, Clock v) {
   const int l = threadIdx.x;
-  if (blockIdx.x == 0) {
-    constexpr int PW = sizeof(Params) / sizeof(uint64_t);
-    static_assert(sizeof(Params) % sizeof(uint64_t) == 0, "the parameters are copied in 8-byte words");
-    const uint64_t* src = reinterpret_cast<const uint64_t*>(&P);
-    for (int i = l; i < PW; i += 256) reinterpret_cast<uint64_t*>(pdev)[i] = src[i];
-    if (l < ATOMIC_SLOTS) {
-      Counters z = {};
-      z.dtmax_bits = (uint64_t)__double_as_longlong(1.e10);
-      cnt[l] = z;
-    }
-    if (l == 0) {
-      v.fatal = 0;
-      v.fatal_seen = 0;
-      *clk = v;
-      *warn_cnt = 0ull;
-    }
+  constexpr int PW = sizeof(Params) / sizeof(uint64_t);
+  static_assert(sizeof(Params) % sizeof(uint64_t) == 0, "the parameters are copied in 8-byte words");
+  const uint64_t* src = reinterpret_cast<const uint64_t*>(&P);
+  for (int i = l; i < PW; i += 256) reinterpret_cast<uint64_t*>(pdev)[i] = src[i];
+  if (l < ATOMIC_SLOTS) {
+    Counters z = {};
+    z.dtmax_bits = (uint64_t)__double_as_longlong(1.e10);
+    cnt[l] = z;
   }
-  const int n3[3] = {P.nx, P.ny, P.nz};
-  const int64_t base[3] = {o0, o1, o2};
-  int64_t r = (int64_t)blockIdx.x * 256 + l;
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const int64_t nf = n3[a] > 1 ? n3[a] - 1 : 1;
-    if (r >= 0 && r < 3 * nf) {
-      const int k = (int)(r / nf), m = (int)(r % nf);
-      tab[base[a] + r] = (m + 1 < n3[a]) ? face_distance(P.d[a], m, k) : 0.;
-    }
-    r -= 3 * nf;
+  if (l == 0) {
+    v.fatal = 0;
+    v.fatal_seen = 0;
+    *clk = v;
+    *warn_cnt = 0ull;
   }
 }
 
@@ -1311,7 +1274,11 @@ int ecg_step_noalloc(const ecg_config* cfg, const void* state_in, void* state_ou
   };
   const size_t o_par = take(sizeof(Params)), o_clk = take(sizeof(Clock));
   const size_t o_cnt = take(sizeof(Counters) * ATOMIC_SLOTS), o_wc = take(sizeof(unsigned long long));
-  const size_t o_tab = take(sizeof(double) * Ly.ntab);
+  // Nine doubles per face of an axis' line that nothing reads: they are part of the size
+  // above which a case is refused.
+  size_t nface = 0;
+  for (int n : {g.nx, g.ny, g.nz}) nface += (size_t)std::max(n - 1, 1);
+  take(3 * sizeof(double) * nface);
   const size_t o_tank = take(sizeof(double) * TANK_REC * (size_t)Ly.ntank);
   const size_t o_ws = (g.order == 2) ? take((size_t)Ly.esize * (size_t)Ly.pitch * (size_t)Ly.nvar) : 0;
   if (used > NOALLOC_SCRATCH_BYTES)
@@ -1321,22 +1288,14 @@ int ecg_step_noalloc(const ecg_config* cfg, const void* state_in, void* state_ou
   int rc = noalloc_scratch(&S);
   if (rc != ECG_OK) return rc;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  double* tab = reinterpret_cast<double*>(S + o_tab);
-  for (int a = 0; a < 3; a++) {
-    P.dcc[a] = tab + Ly.tab_off[a][0];
-    P.dfl[a] = tab + Ly.tab_off[a][1];
-    P.dfr[a] = tab + Ly.tab_off[a][2];
-  }
   P.tank_buf = reinterpret_cast<double*>(S + o_tank);
   P.warn_rec = nullptr;   // warnings are counted, not recorded
   P.warn_cnt = reinterpret_cast<unsigned long long*>(S + o_wc);
   P.warn_cap = 0;
   Clock* clk = reinterpret_cast<Clock*>(S + o_clk);
   Counters* cnt = reinterpret_cast<Counters*>(S + o_cnt);
-  const int64_t ntab = (int64_t)Ly.ntab;
-  hipLaunchKernelGGL(k_noalloc_open, dim3((unsigned)((ntab + 255) / 256)), dim3(256), 0, st, P,
-                     reinterpret_cast<Params*>(S + o_par), clk, cnt, P.warn_cnt, fresh_clock(dt, 0, INFINITY), tab,
-                     (int64_t)Ly.tab_off[0][0], (int64_t)Ly.tab_off[1][0], (int64_t)Ly.tab_off[2][0]);
+  hipLaunchKernelGGL(k_noalloc_open, dim3(1), dim3(256), 0, st, P, reinterpret_cast<Params*>(S + o_par), clk, cnt,
+                     P.warn_cnt, fresh_clock(dt, 0, INFINITY));
   StepLaunch L;
   std::memset(&L, 0, sizeof(L));
   L.pdev = reinterpret_cast<const Params*>(S + o_par);

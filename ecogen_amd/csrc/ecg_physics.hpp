@@ -67,6 +67,30 @@ struct WarnRec {
   double value;        // |f| after the last iteration
 };
 
+// Bounds of the phases' volume fractions and densities (verify_correct): a value past
+// alo / ahi becomes alo_v / ahi_v, a density below 1e-15 rho_v.  One form for both
+// settings of alphaNull: as branches the two forms broke every face's extrapolation into a
+// dozen blocks.
+struct CellFloors {
+  double alo, alo_v, ahi, ahi_v, rho_v;
+  float f_alo, f_alo_v, f_ahi, f_ahi_v, f_rho_v, pad;
+};
+
+// The three distances of interior face m of an axis with cell size d, cells m | m + 1
+// (Element.cpp:77-81, Face.cpp:52-56): which = 0 centre to centre, 1 face to the left
+// centre, 2 face to the right centre.  Centres at (i + 0.5) d (MeshCartesian.cpp:178).
+// The reference's sqrt(x^2 + 0 + 0) of the coordinate difference is |x| exactly: the
+// rounded square's root rounds to |x| unless the square under- or overflows.  The kernels
+// evaluate it where an axis has no single value: a table cost a memory latency at every
+// slope and two, one after the other, at every face (this and the unconditional reads of the
+// second slope: 3D two-phase O2 at 93 x 95 x 91 FP64 442 -> 406 us, 119 x 113 x 117 FP32
+// 376 -> 329).
+__host__ __device__ inline double face_distance(double d, int m, int which) {
+  const double pm = (m + 0.5) * d, pp = (m + 1 + 0.5) * d;
+  const double fp = pm + 0.5 * d;
+  return fabs((which == 0) ? pm - pp : (which == 1) ? fp - pm : fp - pp);
+}
+
 struct Params {
   int nx, ny, nz;
   int64_t ncell;
@@ -82,10 +106,8 @@ struct Params {
   int lim[4];
   int tiles[3];             // tiles per axis
   EosDev eos[4];
-  const double* dcc[3];     // cell-to-cell distance of face m (cells m | m+1)
-  const double* dfl[3];     // face m to its left cell centre
-  const double* dfr[3];     // face m to its right cell centre
-  // Axes whose three distance tables are each one value (the uniform meshes a power-of-two
+  CellFloors floors;
+  // Axes whose three face distances (face_distance) are each one value (the uniform meshes a power-of-two
   // cell count spans exactly): bit a of dist_uniform, the values, and bit a of dcc_pow2 when
   // the cell-to-cell distance is a power of two, so that dividing by it is multiplying by
   // its exact inverse inv_dcc.
@@ -623,15 +645,12 @@ __device__ __forceinline__ void verify_correct(const Params& P, Cell<N, R>& s, i
     s.p[0] = eos_clamp_p<R>(P.eos[0], s.p[0]);
     return;
   }
-  if (P.eps > 1.e-20) {
-    if (s.a[k] < R(0.)) s.a[k] = R(0.);
-    if (s.a[k] > R(1.)) s.a[k] = R(1.);
-    if (s.r[k] <= R(1.e-15)) s.r[k] = R(1.e-15);
-  } else {
-    if (s.a[k] < R(1e-15)) s.a[k] = R(1e-14);
-    if (s.a[k] > R(1.) - R(1e-15)) s.a[k] = R(1.) - R(1e-14);
-    if (s.r[k] < R(1.e-15)) s.r[k] = R(1.e-14);
-  }
+  // With alphaNull: alpha to [0, 1], rho to 1e-15 at least; without: alpha to
+  // [1e-14, 1 - 1e-14] where it passes 1e-15 of the ends, rho below 1e-15 to 1e-14.
+  const CellFloors& q = P.floors;
+  s.a[k] = (s.a[k] < pv<R>(q.alo, q.f_alo)) ? pv<R>(q.alo_v, q.f_alo_v) : s.a[k];
+  s.a[k] = (s.a[k] > pv<R>(q.ahi, q.f_ahi)) ? pv<R>(q.ahi_v, q.f_ahi_v) : s.a[k];
+  s.r[k] = (s.r[k] < R(1.e-15)) ? pv<R>(q.rho_v, q.f_rho_v) : s.r[k];
   s.p[k] = eos_clamp_p<R>(P.eos[k], s.p[k]);
 }
 

@@ -222,18 +222,18 @@ struct FaceDist {
   bool mul;
   __device__ __forceinline__ FaceDist(const Params& P, int m) {
     const bool uni = (P.dist_uniform >> AX) & 1;
-    d = uni ? pv<R>(P.dcc_c[AX], P.f_dcc_c[AX]) : R(P.dcc[AX][m]);
+    d = uni ? pv<R>(P.dcc_c[AX], P.f_dcc_c[AX]) : R(face_distance(P.d[AX], m, 0));
     inv = pv<R>(P.inv_dcc[AX], P.f_inv_dcc[AX]);
     mul = (sizeof(R) == 4) ? uni : (((P.dcc_pow2 >> AX) & 1) != 0);
   }
 };
 template <typename R, int AX>
 __device__ __forceinline__ R face_dfl(const Params& P, int m) {
-  return ((P.dist_uniform >> AX) & 1) ? pv<R>(P.dfl_c[AX], P.f_dfl_c[AX]) : R(P.dfl[AX][m]);
+  return ((P.dist_uniform >> AX) & 1) ? pv<R>(P.dfl_c[AX], P.f_dfl_c[AX]) : R(face_distance(P.d[AX], m, 1));
 }
 template <typename R, int AX>
 __device__ __forceinline__ R face_dfr(const Params& P, int m) {
-  return ((P.dist_uniform >> AX) & 1) ? pv<R>(P.dfr_c[AX], P.f_dfr_c[AX]) : R(P.dfr[AX][m]);
+  return ((P.dist_uniform >> AX) & 1) ? pv<R>(P.dfr_c[AX], P.f_dfr_c[AX]) : R(face_distance(P.d[AX], m, 2));
 }
 
 // Slope of face (L | L+1): (W_R - W_L) / distance, phase variables then velocity;
@@ -270,13 +270,12 @@ __device__ __forceinline__ void slope_vars(const Cell<N, R>& L, const Cell<N, R>
 
 // computeLocalSlopes + limitSlopes + extrapolate + verifyAndCorrectPhase on a
 // uniform Cartesian cell: slope1 is the face's own slope, slope2 the opposite
-// face's slope when that face is interior (boundary faces carry none: slope2
-// and the opposite alpha stay 0).  negate: right cell (changeSign,
+// face's (zero on a boundary face that carries none, as the opposite alpha).  negate: right cell (changeSign,
 // CellInterfaceO2Cartesian.cpp:151-156).  LK >= 0: every limiter of the case is
 // of kind LK (no interface switch to evaluate); LK < 0: kinds from P.lim.  Slope
 // element v at s1[v * S].
 template <int MODEL, int N, int D, typename R, int LK, int S = 1>
-__device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, const R* s1, const R* s2, bool has2,
+__device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, const R* s1, const R* s2,
                                             R aAfter, R aCell, R aOther, R dist, bool negate) {
   int lg = LK, lvf = LK;
   if (LK < 0) {
@@ -290,9 +289,9 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
 #pragma unroll
   for (int k = 0; k < N; k++) {
     R la = R(0.), lr, lp;
-    if (MODEL != M_EULER) { la = limit<R>(lvf, s1[S * v], has2 ? s2[S * v] : R(0.)); v++; }
-    lr = limit<R>(lg, s1[S * v], has2 ? s2[S * v] : R(0.)); v++;
-    lp = limit<R>(lg, s1[S * v], has2 ? s2[S * v] : R(0.)); v++;
+    if (MODEL != M_EULER) { la = limit<R>(lvf, s1[S * v], s2[S * v]); v++; }
+    lr = limit<R>(lg, s1[S * v], s2[S * v]); v++;
+    lp = limit<R>(lg, s1[S * v], s2[S * v]); v++;
     if (negate) { la = -la; lr = -lr; lp = -lp; }
     if (MODEL != M_EULER) b.a[k] += la * dist;
     b.r[k] += lr * dist;
@@ -300,7 +299,7 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
     if (MODEL == M_EULER) {
 #pragma unroll
       for (int d = 0; d < D; d++) {
-        R lu = limit<R>(lg, s1[S * (v + d)], has2 ? s2[S * (v + d)] : R(0.));
+        R lu = limit<R>(lg, s1[S * (v + d)], s2[S * (v + d)]);
         if (negate) lu = lu * R(-1.);
         b.u[d] = b.u[d] + lu * dist;
       }
@@ -310,7 +309,7 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
   if (MODEL != M_EULER) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
-      R lu = limit<R>(lg, s1[S * (v + d)], has2 ? s2[S * (v + d)] : R(0.));
+      R lu = limit<R>(lg, s1[S * (v + d)], s2[S * (v + d)]);
       if (negate) lu = lu * R(-1.);
       b.u[d] = b.u[d] + lu * dist;
     }
@@ -496,6 +495,11 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
           Cell<N, R> cw;
           load_prim<MODEL, N, D, off32<R>()>(P, L.wsrc, cell, cw);
           wall_slope_vars<MODEL, N, D, R, SES>(cw, AX, m < 0 ? pv<R>(P.dwall[AX][0], P.f_dwall[AX][0]) : -pv<R>(P.dwall[AX][1], P.f_dwall[AX][1]), o);
+        } else if (cb < n3[B] && cc < n3[C]) {
+          // No slope beyond the mesh: the limiters read zeros, without a test per variable
+          // (which kept the reads of a record apart, each behind its own mask).
+#pragma unroll
+          for (int v = 0; v < SZ::NS; v++) o[SES * v] = R(0.);
         }
       }
       if (STEPS == STEP_ABC) __syncthreads();
@@ -525,8 +529,8 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
             const R aRR = (LK < 0 && MODEL != M_EULER && hasp)
                               ? alpha0_at<R>(L.wn, (m + 1 <= na - 2) ? cell + 2 * sa : cell + sa)
                               : R(0.);
-            extrapolate<MODEL, N, D, R, LK, SES>(P, bl, s1, s1 - SRS, hasm, aLL, aL, aR, face_dfl<R, AX>(P, m), false);
-            extrapolate<MODEL, N, D, R, LK, SES>(P, br, s1, s1 + SRS, hasp, aRR, aR, aL, face_dfr<R, AX>(P, m), true);
+            extrapolate<MODEL, N, D, R, LK, SES>(P, bl, s1, s1 - SRS, aLL, aL, aR, face_dfl<R, AX>(P, m), false);
+            extrapolate<MODEL, N, D, R, LK, SES>(P, br, s1, s1 + SRS, aRR, aR, aL, face_dfr<R, AX>(P, m), true);
             if constexpr (LK == LK_FULL && MODEL != M_EULER && N == 2) {
               if (P.thinc) {
                 // THINC replaces the extrapolated volume fractions at an interface.
