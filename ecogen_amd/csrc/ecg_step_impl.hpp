@@ -422,6 +422,27 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
   k0 = tz * Tile<D, TK>::Z;
 }
 
+// Accumulators that wait in the thread's own LDS slots while the fluxes are evaluated.  The 3D
+// three-phase FP64 kernels need 187 (first order) and 195 registers and have 168 (three
+// waves per SIMD); what a third of a CU's LDS holds beside the staging, seven and six
+// doubles a thread (nine in 2D), takes the accumulators out of the flux passes, where they had been
+// spilled and reloaded in every pass (256^3 first order: 3186 -> 2692 us a step; two waves
+// per SIMD without spills: 3242).
+template <int MODEL, int N, int D, bool O2, int TK, int LK> constexpr int acc_stash() {
+  if (!(N == 3 && D >= 2 && TK == 8 && LK != LK_FULL)) return 0;
+  const int room = (53760 - 8 * Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) / (256 * 8);
+  return room < 3 * N ? room : 3 * N;
+}
+template <int NS, int N, typename R, class F> __device__ __forceinline__ void each_stashed(ConsAcc<N, R>& acc, F f) {
+  int v = 0;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    if (v < NS) { f(acc.alpha[k].v, v); v++; }
+    if (v < NS) { f(acc.mass[k].v, v); v++; }
+    if (v < NS) { f(acc.energ[k].v, v); v++; }
+  }
+}
+
 // One axis pass (steps A, B, C above) for axis AX with face frame FR, in
 // batches of lines when the staging would exceed lds_batch_bytes.  The small tiles call
 // one step at a time (STEPS) on the axis's own threads, with the barriers between them.
@@ -563,6 +584,9 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
     if (STEPS == STEP_ABC) __syncthreads();
 
     // C. gather: add the lower face, subtract the upper face
+    constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK>();
+    double* st = reinterpret_cast<double*>(lds + SZ::template lds_elems<TK>(O2)) + threadIdx.x;
+    if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { x = st[256 * v]; });
     if ((STEPS & STEP_C) && own_ok && lown / LB == bt) {
       const int t = own[AX] - org[AX];
       const int lb = lown - l0;
@@ -584,6 +608,7 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
         }
       }
     }
+    if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { st[256 * v] = x; });
     if (STEPS == STEP_ABC) __syncthreads();
   }
 }
@@ -852,6 +877,9 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
   }
   ConsAcc<N, R> acc;
 
+  constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK>();
+  double* st = reinterpret_cast<double*>(lds + Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) + tid;
+  if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { st[256 * v] = x; });
   if constexpr (tile_small(TK)) {
     // Waves 0-1 take the x axis, 2-3 y, 4-5 z; the first wave gathers in the faces' order.
     const int grp = __builtin_amdgcn_readfirstlane(tid / pass_threads<TK>());
@@ -874,6 +902,7 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
     if (D >= 2) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
     if (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
   }
+  if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { x = st[256 * v]; });
 
   Cell<N> nw;
   bool relax_now = false, spread_ok = false;
@@ -1215,7 +1244,7 @@ void launch_step_v(const Params& P, const StepLaunchT<R>& L, Clock* clk, Counter
     chunk = (int)std::min<int64_t>(rows, std::max<int64_t>((lines - 4) / T, 1));
     if (chunk < rows && chunk > 1) chunk &= ~1;
   }
-  size_t lds = sizeof(R) * SZ::template lds_elems<TK>(O2);
+  size_t lds = sizeof(R) * SZ::template lds_elems<TK>(O2) + 256 * sizeof(double) * acc_stash<MODEL, N, D, O2, TK, LK>();
   if (LEARN && lds < (size_t)step_block_lds<TK>()) lds = step_block_lds<TK>();
   auto k = k_step<MODEL, N, D, O2, R, LEARN, LK, CAP, TK>;
   // A failure here surfaces as the launch error the caller checks next.
