@@ -453,11 +453,13 @@ __device__ __forceinline__ R limit(int kind, R s1, R s2) {
     out = (prod > R(1e-9)) ? m : R(0.);
   } else if (kind == LIM_VANLEER) {
     R sum = s1 + s2;
-    if ((fabs(sum) > R(1e-6)) && (prod > R(1e-6))) out = qdiv(R(2.) * prod, sum);
+    // The quotient always, then a select: no mask and branch around every variable's.
+    const R q = qdiv(R(2.) * prod, sum);
+    out = ((fabs(sum) > R(1e-6)) && (prod > R(1e-6))) ? q : R(0.);
   } else if (kind == LIM_VANALBADA) {
     R sum = s1 + s2;
-    if ((fabs(s1) > R(1e-6)) && (fabs(s2) > R(1e-6)) && (fabs(sum) > R(1e-6)) && (prod > R(1e-6)))
-      out = qdiv(prod * sum, s1 * s1 + s2 * s2);
+    const R q = qdiv(prod * sum, s1 * s1 + s2 * s2);
+    out = ((fabs(s1) > R(1e-6)) && (fabs(s2) > R(1e-6)) && (fabs(sum) > R(1e-6)) && (prod > R(1e-6))) ? q : R(0.);
   } else if (kind == LIM_SUPERBEE) {
     if (prod > R(1e-6)) out = dmax<R>(dmin<R>(R(2.) * fabs(s1), fabs(s2)), dmin<R>(fabs(s1), R(2.) * fabs(s2)));
     if (s1 < R(0.)) out = -out;

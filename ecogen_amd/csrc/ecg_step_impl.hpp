@@ -268,6 +268,29 @@ __device__ __forceinline__ void slope_vars(const Cell<N, R>& L, const Cell<N, R>
   for (int d = 0; d < D; d++) s[S * v++] = q(Rr.u[d] - L.u[d]);
 }
 
+// Limited slopes of one cell side, kinds known only at run time: one switch for all the
+// variables of a kind (lvf the volume fractions, lg the rest).  A switch per variable had
+// kept the variables apart and broke every
+// face into dozens of blocks (Euler O2 with walls and van Leer, 107 x 109 x 105: 365 -> 326 us).
+template <int MODEL, int N, int D, typename R, int S, bool VF>
+__device__ __forceinline__ void limit_slopes(int kind, const R* s1, const R* s2, R* out) {
+  constexpr int PV = (MODEL == M_EULER) ? 2 : 3 * N;
+  auto all = [&](auto k) {
+#pragma unroll
+    for (int v = 0; v < PV + D; v++)
+      if ((MODEL != M_EULER && v < PV && v % 3 == 0) == VF) out[v] = limit<R>(decltype(k)::value, s1[S * v], s2[S * v]);
+  };
+  switch (kind) {
+    case LIM_THINC:   // minmod where the reconstruction itself does not apply
+    case LIM_MINMOD: all(std::integral_constant<int, LIM_MINMOD>{}); break;
+    case LIM_VANLEER: all(std::integral_constant<int, LIM_VANLEER>{}); break;
+    case LIM_VANALBADA: all(std::integral_constant<int, LIM_VANALBADA>{}); break;
+    case LIM_SUPERBEE: all(std::integral_constant<int, LIM_SUPERBEE>{}); break;
+    case LIM_MC: all(std::integral_constant<int, LIM_MC>{}); break;
+    default: all(std::integral_constant<int, LIM_NONE>{}); break;
+  }
+}
+
 // computeLocalSlopes + limitSlopes + extrapolate + verifyAndCorrectPhase on a
 // uniform Cartesian cell: slope1 is the face's own slope, slope2 the opposite
 // face's (zero on a boundary face that carries none, as the opposite alpha).  negate: right cell (changeSign,
@@ -285,13 +308,21 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
       lg = P.lim[0]; lvf = P.lim[2];
     }
   }
+  R lim[(MODEL == M_EULER ? 2 : 3 * N) + D];
+  if constexpr (LK < 0) {
+    if (MODEL != M_EULER) limit_slopes<MODEL, N, D, R, S, true>(lvf, s1, s2, lim);
+    limit_slopes<MODEL, N, D, R, S, false>(lg, s1, s2, lim);
+  } else {
+#pragma unroll
+    for (int v = 0; v < (MODEL == M_EULER ? 2 : 3 * N) + D; v++) lim[v] = limit<R>(LK, s1[S * v], s2[S * v]);
+  }
   int v = 0;
 #pragma unroll
   for (int k = 0; k < N; k++) {
     R la = R(0.), lr, lp;
-    if (MODEL != M_EULER) { la = limit<R>(lvf, s1[S * v], s2[S * v]); v++; }
-    lr = limit<R>(lg, s1[S * v], s2[S * v]); v++;
-    lp = limit<R>(lg, s1[S * v], s2[S * v]); v++;
+    if (MODEL != M_EULER) { la = lim[v]; v++; }
+    lr = lim[v]; v++;
+    lp = lim[v]; v++;
     if (negate) { la = -la; lr = -lr; lp = -lp; }
     if (MODEL != M_EULER) b.a[k] += la * dist;
     b.r[k] += lr * dist;
@@ -299,7 +330,7 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
     if (MODEL == M_EULER) {
 #pragma unroll
       for (int d = 0; d < D; d++) {
-        R lu = limit<R>(lg, s1[S * (v + d)], s2[S * (v + d)]);
+        R lu = lim[v + d];
         if (negate) lu = lu * R(-1.);
         b.u[d] = b.u[d] + lu * dist;
       }
@@ -309,7 +340,7 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
   if (MODEL != M_EULER) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
-      R lu = limit<R>(lg, s1[S * (v + d)], s2[S * (v + d)]);
+      R lu = lim[v + d];
       if (negate) lu = lu * R(-1.);
       b.u[d] = b.u[d] + lu * dist;
     }
@@ -343,15 +374,18 @@ __device__ __forceinline__ void extrapolate_wall(const Params& P, Cell<N, R>& b,
       lg = P.lim[0]; lvf = P.lim[2];
     }
   }
+  R lim[(MODEL == M_EULER ? 2 : 3 * N) + D];
+  if (MODEL != M_EULER) limit_slopes<MODEL, N, D, R, 1, true>(lvf, s1, s2, lim);
+  limit_slopes<MODEL, N, D, R, 1, false>(lg, s1, s2, lim);
   int v = 0;
 #pragma unroll
   for (int k = 0; k < N; k++) {
-    if (MODEL != M_EULER) { b.a[k] += limit<R>(lvf, s1[v], s2[v]) * dist; v++; }
-    b.r[k] += limit<R>(lg, s1[v], s2[v]) * dist; v++;
-    b.p[k] += limit<R>(lg, s1[v], s2[v]) * dist; v++;
+    if (MODEL != M_EULER) { b.a[k] += lim[v] * dist; v++; }
+    b.r[k] += lim[v] * dist; v++;
+    b.p[k] += lim[v] * dist; v++;
   }
 #pragma unroll
-  for (int d = 0; d < D; d++) b.u[d] = b.u[d] + limit<R>(lg, s1[v + d], s2[v + d]) * dist;
+  for (int d = 0; d < D; d++) b.u[d] = b.u[d] + lim[v + d] * dist;
 }
 
 // A staged face flux: element v at o[v * S].
