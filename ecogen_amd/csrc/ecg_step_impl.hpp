@@ -461,10 +461,11 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
 // waves per SIMD); what a third of a CU's LDS holds beside the staging, seven and six
 // doubles a thread (nine in 2D), takes the accumulators out of the flux passes, where they had been
 // spilled and reloaded in every pass (256^3 first order: 3186 -> 2692 us a step; two waves
-// per SIMD without spills: 3242).
+// per SIMD without spills: 3242).  The first-order FP32 kernel runs five waves that way
+// (step_waves).
 template <int MODEL, int N, int D, bool O2, int TK, int LK> constexpr int acc_stash() {
-  if (!(N == 3 && D >= 2 && TK == 8 && LK != LK_FULL)) return 0;
-  const int room = (53760 - 8 * Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) / (256 * 8);
+  if (!(N == 3 && D >= 2 && (TK == 8 || (TK == 4 && !O2)) && LK != LK_FULL)) return 0;
+  const int room = ((TK == 8 ? 53760 : 32256) - TK * Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) / (256 * 8);
   return room < 3 * N ? room : 3 * N;
 }
 template <int NS, int N, typename R, class F> __device__ __forceinline__ void each_stashed(ConsAcc<N, R>& acc, F f) {
@@ -855,9 +856,11 @@ __device__ __forceinline__ void capture_samples(const SampleSink& K, bool cap, c
 // VGPRs) and in the FP32 LK_FULL kernels; five for the one- and two-phase FP32
 // kernels (96 VGPRs; the 2D and 3D minmod kernels need 76-85 and spill nothing,
 // the 2D first-order cold ones then run six waves; the 2D first-order learned ones
-// need 82-86 and would spill 40 bytes per lane at six); four for the three-phase
-// FP32 kernels (128 VGPRs instead of 131: the 256^3 three-phase step runs 11 %
-// faster than at three; at five they spill too much).
+// need 82-86 and would spill 40 bytes per lane at six); four for the second-order,
+// learned and capture three-phase FP32 kernels (128 VGPRs instead of 131: the 256^3 three-phase step runs 11 %
+// faster than at three; at five they spill too much); five for the first-order
+// three-phase ones, whose accumulators wait in LDS (acc_stash: 89 VGPRs; at 251 x 243 x 257
+// 1205 -> 1166 us a step).
 // LDS of one wave in the learned kernels after the flux passes: the inference's
 // staging (MLP_WAVE_LDS) and two doubles per lane for the start's affine form.
 constexpr int STEP_WAVE_LDS = MLP_WAVE_LDS + 64 * 2 * 8;
@@ -865,7 +868,7 @@ template <int TK> constexpr int step_block_lds() { return tile_cells<TK>() / 64 
 
 template <typename R, int N, int D, bool O2, bool LEARN, int LK>
 constexpr int step_waves() {
-  return (sizeof(R) == 4 && LK != LK_FULL) ? (N <= 2 ? 5 : 4) : 3;
+  return (sizeof(R) == 4 && LK != LK_FULL) ? (N <= 2 || (!O2 && !LEARN) ? 5 : 4) : 3;
 }
 
 // CAP: the instantiation that also captures warm-start training records (cold
@@ -873,7 +876,7 @@ constexpr int step_waves() {
 // always carry it).  Without it the capture path is not compiled: its features
 // and slot arithmetic cost the FP64 benchmark kernel 1 % even when not taken.
 template <int MODEL, int N, int D, bool O2, typename R, bool LEARN, int LK, bool CAP = false, int TK = (int)sizeof(R)>
-__global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, LEARN, LK>())) void k_step(ParamsPtr Pc, StepLaunchT<R> L, Clock* __restrict__ clk,
+__global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, LEARN || CAP, LK>())) void k_step(ParamsPtr Pc, StepLaunchT<R> L, Clock* __restrict__ clk,
                                               Counters* __restrict__ cnt) {
   constexpr bool CAPTURE = !LEARN && MODEL != M_EULER && (CAP || LK == LK_FULL);
   const Params& P = *(const Params*)Pc;
