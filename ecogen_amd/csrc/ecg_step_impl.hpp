@@ -1,6 +1,7 @@
 // Kernel templates of the finite-volume step: face-centric tiles.
 //
-// A 256-thread block owns a tile of cells (256 x 1, 16 x 16 or 16 x 4 x 4) and
+// A 256-thread block owns a tile of cells (256 x 1, 16 x 16, 16 x 4 x 4 or 8 x 8 x 4; small
+// meshes take tiles of 64 cells) and
 // walks the axes in the reference's face-creation order (X, Y, Z; then the
 // boundary faces X-, X+, Y-, Y+, Z-, Z+ of MeshCartesian.cpp:283-557).  For
 // each axis it

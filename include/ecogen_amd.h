@@ -248,7 +248,7 @@ int ecg_set_time(ecg_ctx* ctx, double t, double dt, int64_t iteration);
  * library's layout (the variables above, each over pitch = ncell rounded up to 64
  * elements; double for ECG_FP64, float for ECG_FP32_RELAX64) and gets the state after
  * one step of size dt in state_out.  Everything else (parameters, clock, counters,
- * distance tables, inlet-tank records, the second-order predicted state) lives in a
+ * inlet-tank records, the second-order predicted state) lives in a
  * fixed 64 MiB device array of the library, one per GPU, held until the process ends;
  * a case that needs more is refused with ECG_E_ARG.  The call allocates nothing, runs
  * on `stream` (NULL: the null stream) and waits for it; *dtmax_out receives dtMax.
