@@ -60,3 +60,30 @@ def test_both_tile_kinds_match_the_oracle(name, side, precision):
            if case["model"] != "euler" else s[names.index("rho")] for s in (sg, so)]
     assert np.all(np.isfinite(sg))
     assert rel_l1(*mix) <= 1e-5
+
+
+# Split launches of the ordinary tiles (a launch of n tile rows of T lines reads n T + 4 lines), and of
+# small ones in 2D (T = 8): one row, two, uneven rests.
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,mesh,lines", [("ueq2_3d_o2", (65, 31, 30), 8), ("ueq2_3d_o2", (65, 31, 30), 13),
+                                             ("ueq2_3d_o2", (65, 31, 30), 24), ("pueq_2d_o2", (257, 243, 1), 20),
+                                             ("pueq_2d_o2", (257, 243, 1), 53), ("pueq_2d_o2", (100, 90, 1), 12),
+                                             ("pueq_2d_o2", (100, 90, 1), 29)])
+def test_split_launches_of_both_tile_kinds(name, mesh, lines):
+    from ecogen_amd import Solver, library
+    case = dict(CASES[name], precision="fp32")
+    case["nx"], case["ny"], case["nz"] = mesh
+    line_cells = mesh[0] * mesh[1] if mesh[2] > 1 else mesh[0]
+    out = []
+    for span in (1 << 32, lines * line_cells * 4):
+        prev = library().ecg_set_step_span(span)
+        try:
+            g = Solver(case)
+            dt = 1.e-15
+            for _ in range(3):
+                dt = case["cfl"] * g.step(dt)[0]
+            out.append((dt, g.get_state()))
+        finally:
+            library().ecg_set_step_span(prev)
+    assert out[0][0] == out[1][0]
+    np.testing.assert_array_equal(out[1][1], out[0][1])
