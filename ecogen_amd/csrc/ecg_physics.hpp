@@ -193,7 +193,8 @@ __device__ __forceinline__ float fpow(float x, float y) { return __builtin_amdgc
 // quotient, with bit-identical results: the sequence's pre-scaling and fix-up
 // act only on operands within a few binades of overflow or underflow and on
 // zeros, infinities and NaNs, none of which the face and cell arithmetic divides
-// by (densities and masses are floored, wave-speed differences are nonzero).
+// by (multiphase densities and masses are floored, wave-speed differences are nonzero; Euler's
+// density is not, and its quotients take the fix-up: derive, build_prim).
 __device__ __forceinline__ double rcp_ieee(double b) {
   const double r0 = __builtin_amdgcn_rcp(b);
   const double r1 = fma(r0, fma(-b, r0, 1.), r0);
@@ -219,6 +220,16 @@ template <> struct Quot<float> {
   float rb;
   __device__ __forceinline__ explicit Quot(float d) : rb(__builtin_amdgcn_rcpf(d)) {}
   __device__ __forceinline__ float operator()(float a) const { return a * rb; }
+};
+// Quotients by one divisor that may be zero, infinite, NaN or subnormal (Euler densities carry
+// no floor): tiny divisors are scaled into the reciprocal's range, exactly, and the hardware's
+// fix-up gives the special values.
+struct QuotFull {
+  double s, b, rb;
+  __device__ __forceinline__ explicit QuotFull(double d) : s(fabs(d) < 1.e-290 ? 0x1p512 : 1.), b(d * s), rb(rcp_ieee(b)) {}
+  __device__ __forceinline__ double operator()(double a) const {
+    return __builtin_amdgcn_div_fixup(div_ieee(a, b, rb), b, a) * s;
+  }
 };
 // The square root as the device's sequence forms it (reciprocal square-root
 // estimate, one Goldschmidt step on the root and its half-reciprocal, two Newton
@@ -563,16 +574,16 @@ __device__ __forceinline__ void derive(const Params& P, Cell<N, R>& s, bool rebu
   const R eps = pv<R>(P.eps, P.f_eps);
   if (MODEL == M_EULER) {
     if constexpr (sizeof(R) == 8) {
-      // One reciprocal of the density for the energy and the squared sound speed; the
-      // lean square root inside its range (Euler pressures carry no floor: anything else,
-      // a negative or NaN argument included, takes the library's).
+      // One reciprocal of the density for the energy and the squared sound speed.  Euler
+      // densities and pressures carry no floor: a vacuum's sound speed is infinite, which makes the
+      // step's dtMax zero, so the hardware's fix-up gives the quotient by a zero density (one whose
+      // reciprocal overflows counts as zero) and the library's root the special values.  (The
+      // lean root with a test of its range before the library's: 121 x 119 x 117 first order 96
+      // us a step, this 88; with second-order walls 357 / 343.)
       const EosDev& q = P.eos[0];
-      const double rr = dmax<double>(s.r[0], eps), ir = rcp_ieee(rr);
+      const double rr = dmax<double>(s.r[0], eps), ir = rcp_ieee(rr), cn = q.g * (s.p[0] + q.pinf);
       s.e[0] = div_ieee(div_ieee(s.p[0] + q.gpinf, q.gm1, q.mixinv), rr, ir) + q.eref;
-      const double c2 = div_ieee(q.g * (s.p[0] + q.pinf), rr, ir);
-      double c = sqrt_pos(c2);
-      if (!(c2 > 1.e-200 && c2 < 1.e200)) c = sqrt(c2);
-      s.c[0] = c;
+      s.c[0] = sqrt(__builtin_amdgcn_div_fixup(div_ieee(cn, rr, ir), rr < 0x1p-1024 ? 0. : rr, cn));
     } else {
       s.e[0] = eos_energy<R>(P.eos[0], eps, s.r[0], s.p[0]);
       s.c[0] = eos_sound<R>(P.eos[0], eps, s.r[0], s.p[0]);
@@ -1204,12 +1215,13 @@ __device__ __forceinline__ void build_prim(const Params& P, Cons<N>& A, Cell<N>&
   if (MODEL == M_EULER) {
     const double m = A.mass[0];
     s.r[0] = m;
-    const double im = rcp_ieee(m);   // one reciprocal for the four quotients by the density
-    s.u[0] = div_ieee(A.mom[0], m, im); s.u[1] = div_ieee(A.mom[1], m, im); s.u[2] = div_ieee(A.mom[2], m, im);
+    // One reciprocal for the four quotients by the density.
+    const QuotFull q(m);
+    s.u[0] = q(A.mom[0]); s.u[1] = q(A.mom[1]); s.u[2] = q(A.mom[2]);
+    s.E = q(A.energM);
     if (fabs(s.u[0]) < 1.e-8) s.u[0] = 0.;
     if (fabs(s.u[1]) < 1.e-8) s.u[1] = 0.;
     if (fabs(s.u[2]) < 1.e-8) s.u[2] = 0.;
-    s.E = div_ieee(A.energM, m, im);
     const double e = s.E - 0.5 * sqn3<double>(s.u);
     s.e[0] = e;
     s.p[0] = eos_pressure<double>(P.eos[0], m, e);
