@@ -724,6 +724,16 @@ static void unpack_state(const ecg_ctx* c, double* const* soa, const unsigned ch
   }
 }
 
+// Whether two of the caller's arrays share memory: the later variable's values then stand.
+static bool arrays_overlap(const ecg_ctx* c, double* const* soa) {
+  uintptr_t at[3 * ECG_MAX_PHASES + 3];
+  for (int v = 0; v < c->nvar; v++) at[v] = reinterpret_cast<uintptr_t>(soa[v]);
+  std::sort(at, at + c->nvar);
+  for (int v = 1; v < c->nvar; v++)
+    if (at[v] - at[v - 1] < sizeof(double) * (uintptr_t)c->ncell) return true;
+  return false;
+}
+
 // The state through pinned buffers of 1 MB: large states by up to eight threads, each with a
 // buffer of its own, that copy and unpack every eighth piece.  The host side is the bound:
 // the caller's arrays are usually fresh pages, and one thread converting floats into them
@@ -731,7 +741,9 @@ static void unpack_state(const ecg_ctx* c, double* const* soa, const unsigned ch
 static int download_state(ecg_ctx* c, double* const* soa) {
   const int64_t total = c->pitch * c->nvar, piece = std::min<int64_t>(total, (int64_t(1) << 20) / c->esize);
   const int64_t npiece = (total + piece - 1) / piece;
-  const int team = (int)std::min<int64_t>(std::min(8u, std::max(1u, std::thread::hardware_concurrency())), npiece);
+  const int team = arrays_overlap(c, soa)   // in order
+                       ? 1
+                       : (int)std::min<int64_t>(std::min(8u, std::max(1u, std::thread::hardware_concurrency())), npiece);
   for (int b = 0; b < team; b++) {
     if (!c->bounce[b]) HIPCHK(hipHostMalloc((void**)&c->bounce[b], (size_t)piece * c->esize, hipHostMallocDefault));
     if (!c->bounce_ev[b]) HIPCHK(hipEventCreateWithFlags(&c->bounce_ev[b], hipEventDisableTiming));
