@@ -724,6 +724,18 @@ static void unpack_state(const ecg_ctx* c, double* const* soa, const unsigned ch
   }
 }
 
+// Whether p is memory that the device copies to directly: page-locked, or the device's own or
+// managed memory (*device), which the host threads need not reach.
+static bool device_reachable(const void* p, bool* device) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();   // an address the runtime does not know: ordinary host memory
+    return false;
+  }
+  *device = at.type == hipMemoryTypeManaged || at.type == hipMemoryTypeDevice;
+  return *device || at.type == hipMemoryTypeHost;
+}
+
 // Whether two of the caller's arrays share memory: the later variable's values then stand.
 static bool arrays_overlap(const ecg_ctx* c, double* const* soa) {
   uintptr_t at[3 * ECG_MAX_PHASES + 3];
@@ -734,11 +746,29 @@ static bool arrays_overlap(const ecg_ctx* c, double* const* soa) {
   return false;
 }
 
+// One variable after the other, by the runtime's own copies (FP64).
+static int download_plain(ecg_ctx* c, double* const* soa) {
+  for (int v = 0; v < c->nvar; v++) {
+    const double* src = static_cast<const double*>(c->W[c->cur]) + (size_t)v * c->pitch;
+    HIPCHK(hipMemcpyAsync(soa[v], src, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->stream));
+  }
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return ECG_OK;
+}
+
 // The state through pinned buffers of 1 MB: large states by up to eight threads, each with a
 // buffer of its own, that copy and unpack every eighth piece.  The host side is the bound:
 // the caller's arrays are usually fresh pages, and one thread converting floats into them
-// took 8 ms for the ten variables of a 104^3 mesh, half of a 32-step run.
+// took 8 ms for the ten variables of a 104^3 mesh, half of a 32-step run.  FP64 states of
+// 2 MB and more go straight into page-locked arrays (eight variables, through the buffers /
+// straight, ms: 128^2 (1 MB) 0.070 / 0.104, 181^2 0.115 / 0.115, 512^2 0.67 / 0.41, 160^3 10.4 /
+// 5.8), and any into device memory.
 static int download_state(ecg_ctx* c, double* const* soa) {
+  const bool large = (int64_t)c->esize * c->pitch * c->nvar >= (int64_t(2) << 20);
+  for (int v = 0; v < c->nvar && c->esize == 8; v++) {
+    bool device = false;
+    if (device_reachable(soa[v], &device) && (large || device)) return download_plain(c, soa);
+  }
   const int64_t total = c->pitch * c->nvar, piece = std::min<int64_t>(total, (int64_t(1) << 20) / c->esize);
   const int64_t npiece = (total + piece - 1) / piece;
   const int team = arrays_overlap(c, soa)   // in order

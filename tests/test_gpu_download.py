@@ -1,12 +1,17 @@
 """ecg_download_state into every kind of array a caller may hold (needs a GPU).  The state itself is
 what ecg_upload_state stored."""
 import ctypes as C
+import os
+import subprocess
+import sys
+import textwrap
 
 import numpy as np
 import pytest
 
 from ecogen_amd.case import IG_AIR, SG_WATER
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 DP = C.POINTER(C.c_double)
 
 
@@ -41,3 +46,54 @@ def test_arrays_that_share_memory_hold_the_last_variable(mesh, precision):
         assert _download(s, [first] + [one] * (s.nvar - 1)) == 0
         np.testing.assert_array_equal(first, st[0])
         np.testing.assert_array_equal(one, st[-1])
+
+
+# A library that stands before the HIP runtime in the child's symbol order and counts the copies.
+SHIM = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+static void* sym(const char* n) { return dlsym(dlopen("libamdhip64.so.7", RTLD_LAZY), n); }
+size_t copied_to_caller, copied_elsewhere;
+char *caller_lo, *caller_hi;
+int hipMemcpyAsync(void* d, const void* s, size_t n, int k, void* st) {
+  if (k == 2) { if ((char*)d >= caller_lo && (char*)d < caller_hi) copied_to_caller += n; else copied_elsewhere += n; }
+  return ((int (*)(void*, const void*, size_t, int, void*))sym("hipMemcpyAsync"))(d, s, n, k, st);
+}
+"""
+CHILD = textwrap.dedent("""
+    import ctypes as C, sys
+    import numpy as np
+    sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+    shim = C.CDLL(sys.argv[2], mode=C.RTLD_GLOBAL)
+    var = lambda n, t=C.c_int: t.in_dll(shim, n)
+    from test_gpu_download import _download, _solver
+    hip = C.CDLL("libamdhip64.so.7")
+    hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    for precision in ("fp64", "fp32"):
+        s, st = _solver(701, 683, precision)
+        p = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(p), st.nbytes, 0) == 0
+        locked = np.frombuffer((C.c_char * st.nbytes).from_address(p.value)).reshape(st.shape)
+        locked[:] = 0
+        var("caller_lo", C.c_void_p).value, var("caller_hi", C.c_void_p).value = p.value, p.value + st.nbytes
+        to, other = var("copied_to_caller", C.c_size_t), var("copied_elsewhere", C.c_size_t)
+        to.value = other.value = 0
+        print("[download] page-locked", precision, flush=True)
+        assert _download(s, list(locked)) == 0 and np.array_equal(locked, st)
+        if precision == "fp64":   # no detour through the staging buffers
+            assert to.value == s.nvar * s.ncell * 8, (to.value, other.value)
+        mixed = [locked[v] if v % 2 else np.zeros(s.ncell) for v in range(s.nvar)]
+        locked[:] = 0
+        assert _download(s, mixed) == 0 and all(np.array_equal(a, b) for a, b in zip(mixed, st))
+        s.close()
+    print("ok")
+""")
+
+
+@pytest.mark.gpu
+def test_page_locked_arrays(tmp_path):
+    src, lib = tmp_path / "shim.c", tmp_path / "shim.so"
+    src.write_text(SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", str(src), "-o", str(lib), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-u", "-c", CHILD, ROOT, str(lib)], capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and r.stdout.rstrip().endswith("ok"), r.stdout + r.stderr
