@@ -8,7 +8,9 @@
 #include <cstdio>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -746,13 +748,22 @@ static bool arrays_overlap(const ecg_ctx* c, double* const* soa) {
   return false;
 }
 
-// One variable after the other, by the runtime's own copies (FP64).
+// One variable after the other, by the runtime's own copies.
 static int download_plain(ecg_ctx* c, double* const* soa) {
-  for (int v = 0; v < c->nvar; v++) {
-    const double* src = static_cast<const double*>(c->W[c->cur]) + (size_t)v * c->pitch;
-    HIPCHK(hipMemcpyAsync(soa[v], src, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->stream));
+  std::unique_ptr<float[]> tmp;
+  if (c->esize == 4) {
+    tmp.reset(new (std::nothrow) float[c->ncell]);
+    if (!tmp) return fail(ECG_E_ARG, "no host memory for the state's conversion");
   }
-  HIPCHK(hipStreamSynchronize(c->stream));
+  for (int v = 0; v < c->nvar; v++) {
+    const char* src = static_cast<const char*>(c->W[c->cur]) + (size_t)v * c->pitch * c->esize;
+    void* dst = c->esize == 8 ? static_cast<void*>(soa[v]) : tmp.get();
+    HIPCHK(hipMemcpyAsync(dst, src, (size_t)c->esize * c->ncell, hipMemcpyDeviceToHost, c->stream));
+    if (c->esize == 8 && v + 1 < c->nvar) continue;
+    HIPCHK(hipStreamSynchronize(c->stream));
+    if (c->esize == 4)
+      for (int64_t i = 0; i < c->ncell; i++) soa[v][i] = (double)tmp[i];
+  }
   return ECG_OK;
 }
 
@@ -762,7 +773,8 @@ static int download_plain(ecg_ctx* c, double* const* soa) {
 // took 8 ms for the ten variables of a 104^3 mesh, half of a 32-step run.  FP64 states of
 // 2 MB and more go straight into page-locked arrays (eight variables, through the buffers /
 // straight, ms: 128^2 (1 MB) 0.070 / 0.104, 181^2 0.115 / 0.115, 512^2 0.67 / 0.41, 160^3 10.4 /
-// 5.8), and any into device memory.
+// 5.8), and any into device memory.  Where page-locked memory is refused, as many threads
+// as got a buffer share the pieces, and without any the runtime copies.
 static int download_state(ecg_ctx* c, double* const* soa) {
   const bool large = (int64_t)c->esize * c->pitch * c->nvar >= (int64_t(2) << 20);
   for (int v = 0; v < c->nvar && c->esize == 8; v++) {
@@ -771,13 +783,21 @@ static int download_state(ecg_ctx* c, double* const* soa) {
   }
   const int64_t total = c->pitch * c->nvar, piece = std::min<int64_t>(total, (int64_t(1) << 20) / c->esize);
   const int64_t npiece = (total + piece - 1) / piece;
-  const int team = arrays_overlap(c, soa)   // in order
+  const int want = arrays_overlap(c, soa)   // in order
                        ? 1
                        : (int)std::min<int64_t>(std::min(8u, std::max(1u, std::thread::hardware_concurrency())), npiece);
-  for (int b = 0; b < team; b++) {
-    if (!c->bounce[b]) HIPCHK(hipHostMalloc((void**)&c->bounce[b], (size_t)piece * c->esize, hipHostMallocDefault));
-    if (!c->bounce_ev[b]) HIPCHK(hipEventCreateWithFlags(&c->bounce_ev[b], hipEventDisableTiming));
+  int team = 0;
+  while (team < want) {
+    if (!c->bounce_ev[team] && hipEventCreateWithFlags(&c->bounce_ev[team], hipEventDisableTiming) != hipSuccess) break;
+    if (!c->bounce[team] &&
+        hipHostMalloc((void**)&c->bounce[team], (size_t)piece * c->esize, hipHostMallocDefault) != hipSuccess) {
+      c->bounce[team] = nullptr;
+      break;
+    }
+    team++;
   }
+  if (team < want) (void)hipGetLastError();
+  if (team == 0) return download_plain(c, soa);
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   const unsigned char* src = static_cast<const unsigned char*>(c->W[c->cur]);

@@ -1,5 +1,5 @@
-"""ecg_download_state into every kind of array a caller may hold (needs a GPU).  The state itself is
-what ecg_upload_state stored."""
+"""ecg_download_state into every kind of array a caller may hold, and where page-locked memory is
+refused (needs a GPU).  The state itself is what ecg_upload_state stored."""
 import ctypes as C
 import os
 import subprocess
@@ -48,13 +48,20 @@ def test_arrays_that_share_memory_hold_the_last_variable(mesh, precision):
         np.testing.assert_array_equal(one, st[-1])
 
 
-# A library that stands before the HIP runtime in the child's symbol order and counts the copies.
+# A library that stands before the HIP runtime in the child's symbol order: it counts the copies
+# and, when told to, refuses page-locked allocations of 4 KB or more, the runtime's own answer
+# when there is no such memory left.
 SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 static void* sym(const char* n) { return dlsym(dlopen("libamdhip64.so.7", RTLD_LAZY), n); }
+int refuse, refused;
 size_t copied_to_caller, copied_elsewhere;
 char *caller_lo, *caller_hi;
+int hipHostMalloc(void** p, size_t n, unsigned f) {
+  if (refuse && n >= 4096) { refused++; if (refused > refuse - 1) return 2; }
+  return ((int (*)(void**, size_t, unsigned))sym("hipHostMalloc"))(p, n, f);
+}
 int hipMemcpyAsync(void* d, const void* s, size_t n, int k, void* st) {
   if (k == 2) { if ((char*)d >= caller_lo && (char*)d < caller_hi) copied_to_caller += n; else copied_elsewhere += n; }
   return ((int (*)(void*, const void*, size_t, int, void*))sym("hipMemcpyAsync"))(d, s, n, k, st);
@@ -70,6 +77,13 @@ CHILD = textwrap.dedent("""
     hip = C.CDLL("libamdhip64.so.7")
     hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
     for precision in ("fp64", "fp32"):
+        for refuse in (1, 4):   # from the first buffer on, from the fourth on
+            s, st = _solver(701, 683, precision)
+            var("refused").value, var("refuse").value = 0, refuse
+            print("[download] refused", precision, refuse, flush=True)
+            assert np.array_equal(s.get_state(), st) and var("refused").value >= 1
+            var("refuse").value = 0
+            s.close()
         s, st = _solver(701, 683, precision)
         p = C.c_void_p()
         assert hip.hipHostMalloc(C.byref(p), st.nbytes, 0) == 0
@@ -91,7 +105,7 @@ CHILD = textwrap.dedent("""
 
 
 @pytest.mark.gpu
-def test_page_locked_arrays(tmp_path):
+def test_refused_staging_and_page_locked_arrays(tmp_path):
     src, lib = tmp_path / "shim.c", tmp_path / "shim.so"
     src.write_text(SHIM)
     subprocess.run(["gcc", "-shared", "-fPIC", "-O1", str(src), "-o", str(lib), "-ldl"], check=True)
