@@ -92,6 +92,7 @@ SIGNATURES = {
     "ecg_exp": (C.c_double, [C.c_double]),
     "ecg_pow": (C.c_double, [C.c_double, C.c_double]),
     "ecg_log": (C.c_double, [C.c_double]),
+    "ecg_tile_of_block": (C.c_int, [C.POINTER(EcgConfig), C.c_int, C.c_int]),
     "ecg_set_step_span": (C.c_int64, [C.c_int64]),
     "ecg_set_time": (C.c_int, [C.c_void_p, C.c_double, C.c_double, C.c_int64]),
     "ecg_output_open": (C.c_void_p, [C.c_char_p, C.c_char_p, C.c_char_p]),

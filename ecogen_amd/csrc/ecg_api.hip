@@ -1039,6 +1039,12 @@ int ecg_run(ecg_ctx* c, int64_t max_iter, double t_end, ecg_step_stats* st) {
   return run_clock(c, fresh_clock(1.e-15, max_iter, max_iter > 0 ? INFINITY : t_end), max_iter, st);
 }
 
+int ecg_tile_of_block(const ecg_config* cfg, int ntiles, int block) {
+  if (!cfg || ntiles < 1 || block < 0 || block >= ntiles) return fail(ECG_E_ARG, "block outside the launch");
+  const int d = (cfg->nx > 1) + (cfg->ny > 1) + (cfg->nz > 1);
+  return xcd_tile(ntiles, block, tile_run(cfg->model, cfg->nph, d, cfg->precision == ECG_FP32_LEARNED, ntiles));
+}
+
 double ecg_exp(double x) { return exp_cr(x); }
 double ecg_log(double x) { return log_pos(x); }
 double ecg_pow(double x, double y) { return pow_cr(x, y); }

@@ -65,6 +65,38 @@ struct StepLaunchT {
 typedef void (*step_fn)(const Params& P, const StepLaunch& L, Clock* clk, Counters* cnt, hipStream_t s);
 typedef void (*fill_fn)(const Params& P, const DomainDev* doms, int ndom, void* w, hipStream_t s);
 
+// Tile that block `block` of a launch over nb tiles works on.  The chip hands block i to XCD
+// i % 8, and neighbouring tiles share halo lines in an XCD's L2.  run = 0: one range of nb / 8
+// consecutive tiles per XCD (the first nb % 8 one tile longer).  run > 0: runs of that many
+// tiles dealt to the XCDs in turn, what is left over in eight ranges, so that a region whose
+// cells cost more (a shock's relaxation) is shared by all XCDs.
+__host__ __device__ inline int xcd_tile(int nb, int block, int run) {
+  const int xcd = block & 7, full = run > 0 ? nb / (8 * run) * (8 * run) : 0;
+  if (run > 0 && block < full) {
+    const int i = block >> 3;
+    return (i / run * 8 + xcd) * run + i % run;
+  }
+  const int rest = nb - full, rem = rest & 7;
+  return full + xcd * (rest >> 3) + (xcd < rem ? xcd : rem) + ((block - full) >> 3);
+}
+
+// Tiles per run of xcd_tile for a step launch over nb tiles of 256 cells, of a case with n phases
+// in d dimensions; 0: one range per XCD.  Ranges share the most halos, and where every tile costs
+// the same they are the fastest: Euler 3D O1 FP64 at 121 x 119 x 117 97 us a step, dealt singly 157.
+// A two-phase step's relaxation makes the tiles around a shock and the interfaces cost a multiple
+// of the others, and ranges leave them to one or two XCDs: 2D O1 FP64 at 701 x 683 (1892 tiles) 73
+// us in ranges, 64 dealt singly, 62 in runs of 32 (2048^2 379 / 363 / 367); O2 FP32 113 / 110 / 99
+// (1361 x 1283 233 / 281 / 213).  In 3D runs of 64 keep the x and y neighbours together: O2 FP64
+// at 93 x 95 x 91 449 / 472 / 423, FP32 222 / 239 / 204; beyond 6144 tiles (eight rounds of three
+// blocks a CU) the costs even out within a range, and its shared z halos win (O1 FP32 at 119 x
+// 113 x 117 144 us, in runs of 64 150).  Three-phase steps gain nothing (2D O1 FP64 at 907 x 883
+// 109 us in ranges and in runs), nor do learned ones in 3D, whose relaxations are short (O1 at 101 x
+// 99 x 97 112 us in ranges, 122 in runs of 32), nor the small tiles, all resident at once.
+__host__ __device__ constexpr int tile_run(int model, int n, int d, bool learned, int nb) {
+  if (model == M_EULER || n != 2 || d == 1) return 0;
+  return d == 2 ? 32 : !learned && nb <= 6144 ? 64 : 0;
+}
+
 // Tile extents (cells per block along x, y, z) for a problem dimension and state element size.
 void tile_extent(int dim, int esize, int t[3]);
 

@@ -423,20 +423,16 @@ __device__ __forceinline__ void flux_from_lds(const R* o, Flux<N, R>& F) {
 }
 
 // Tile origin of the block among the launch's tile rows (row0, nrows of the
-// outermost axis), XCD-aware: each of the 8 XCDs receives a contiguous range of tiles
-// (neighbours share an L2).
-template <int D, int TK>
+// outermost axis).
+template <int MODEL, int N, int D, bool LEARN, int TK>
 __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows, int& i0, int& j0, int& k0) {
   const int tiles1 = tile_small(TK) ? (P.ny + Tile<D, TK>::Y - 1) / Tile<D, TK>::Y : P.tiles[1];
   const int t0 = (D == 1) ? nrows : tile_small(TK) ? (P.nx + Tile<D, TK>::X - 1) / Tile<D, TK>::X : P.tiles[0];
   const int t1 = (D == 2) ? nrows : (D == 3) ? tiles1 : 1;
   const int nb = t0 * t1 * ((D == 3) ? nrows : 1);
-  // XCD x runs the blocks x, x + 8, ...: it takes a run of nb / 8 tiles, the first nb % 8
-  // XCDs one more.  (Ranges only where 8 divides nb left the others dealt out singly, with
-  // every halo fetched by several L2s: 2D two-phase O2 FP32 at 1361 x 1283, 6966 tiles, 310
-  // -> 236 us a step; Euler with walls at 107 x 109 x 105, 5292 tiles, 390 -> 365.)
-  const int xcd = blockIdx.x & 7, rem = nb & 7;
-  const int b = xcd * (nb >> 3) + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  constexpr int RUN = tile_small(TK) ? 0 : tile_run(MODEL, N, D, LEARN, 0);   // of the launches in runs
+  const int b = (RUN > 0 && tile_run(MODEL, N, D, LEARN, nb) > 0) ? xcd_tile(nb, blockIdx.x, RUN)
+                                                                  : xcd_tile(nb, blockIdx.x, 0);
   int tx = b % t0;
   const int rest = b / t0;
   int ty = rest % t1;
@@ -889,7 +885,7 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
   if (clk->done) return;
   const double dt = clk->dt;
   int org[3];
-  tile_origin<D, TK>(P, L.row0, L.nrows, org[0], org[1], org[2]);
+  tile_origin<MODEL, N, D, LEARN, TK>(P, L.row0, L.nrows, org[0], org[1], org[2]);
   const int tid = threadIdx.x;
   int own[3];
   own[0] = org[0] + tid % Tile<D, TK>::X;

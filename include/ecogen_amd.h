@@ -177,6 +177,9 @@ double ecg_exp(double x);
  * arguments give what the C library's log gives; the same code on the host and the
  * device. */
 double ecg_log(double x);
+/* Tile that block `block` of a step launch over `ntiles` tiles of 256 cells of the case works on
+ * (the kernels' own order, for tests): a permutation of 0 .. ntiles - 1. */
+int ecg_tile_of_block(const ecg_config* cfg, int ntiles, int block);
 /* The pow the full-featured FP64 kernels use in the star-state isentropes
  * (EosSG.cpp:129-132 calls std::pow): correctly rounded for a positive finite base and
  * a result between 2^-1010 and 2^1010, the library's pow otherwise; the same code on
