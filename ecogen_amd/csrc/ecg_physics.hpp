@@ -1287,15 +1287,24 @@ struct NewtonState { double p, f, df; int it; };
 // Newton evaluations of f = sum_k alpha_k rho_k / rho_k(p) - 1 on the cell's
 // pre-relaxation phases (s, unchanged) from st until |f| <= 1e-10 or st.it reaches
 // maxit; akS / rkS receive the phases at the last evaluation.
-template <int N>
+// The first evaluation forms f' only where another iterate follows: nearly every relaxation is
+// settled there (1.03 evaluations per relaxation on the 512^3 two-phase case), and the
+// derivative is two quotients per phase.  A settled st keeps an unread f'.  With BESIDE the
+// evaluations after it form f' beside f, in a copy of their own: a lane behind a shock takes
+// tens of them, and its chain is what a small mesh's step waits for.  Two-phase second
+// order, us a step with f' on demand throughout / beside: 96^2 69.0 / 65.2, 24^3 76.4 / 72.9;
+// the 3D FP64 kernel of the finite-rate relaxation spills 186 / 41 VGPRs and takes 280 / 254
+// at 77 x 75 x 73.  The copy costs three-phase (24^3 18.1 / 18.6) and learned kernels
+// (2D walls 94 / 96) more than it saves.
+template <int N, bool BESIDE = (N == 2)>
 __device__ __forceinline__ void newton_resume(const Params& P, const Cell<N>& s, NewtonState& st, double* akS,
                                               double* rkS, int maxit) {
-  do {
+  auto evaluate = [&](bool beside) {
     st.it++;
     st.p -= div1(st.f, st.df);
 #pragma unroll
     for (int k = 0; k < N; k++) st.p = eos_clamp_p<double>(P.eos[k], st.p);
-    double f = -1.;
+    double f = -1., df = 0.;
 #pragma unroll
     for (int k = 0; k < N; k++) {
       rkS[k] = eos_rho_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], st.p);
@@ -1303,11 +1312,7 @@ __device__ __forceinline__ void newton_resume(const Params& P, const Cell<N>& s,
       f += akS[k];
     }
     st.f = f;
-    // f' only where another iterate follows: nearly every relaxation is settled by its
-    // first evaluation (1.03 evaluations per relaxation on the 512^3 two-phase case), and
-    // the derivative is two quotients per phase.  A settled st keeps an unread f'.
-    if (fabs(f) > 1e-10) {
-      double df = 0.;
+    if (beside || fabs(f) > 1e-10) {
 #pragma unroll
       for (int k = 0; k < N; k++) {
         const double drhodp = eos_drhodp_pfinal(P.eos[k], P.eps, s.p[k], s.r[k], st.p);
@@ -1315,7 +1320,14 @@ __device__ __forceinline__ void newton_resume(const Params& P, const Cell<N>& s,
       }
       st.df = df;
     }
-  } while (fabs(st.f) > 1e-10 && st.it < maxit);
+  };
+  if constexpr (BESIDE) {
+    evaluate(false);
+    while (fabs(st.f) > 1e-10 && st.it < maxit) evaluate(true);
+  } else {
+    do evaluate(false);
+    while (fabs(st.f) > 1e-10 && st.it < maxit);
+  }
 }
 
 // Outcome flags of a relaxation's Newton solve: RELAX_FAIL when it spent its 100

@@ -1005,7 +1005,7 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
         if (relax_now) {
           double akS[N], rkS[N];
           NewtonState s1{relax_guess<N>(nw), 0., 1., 0};
-          newton_resume<N>(P, nw, s1, akS, rkS, 1);
+          newton_resume<N, false>(P, nw, s1, akS, rkS, 1);
           if (fabs(s1.f) <= 1e-10) {
             relaxed1 = true;
             carry = s1.f;
@@ -1061,7 +1061,7 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
           const double guess = ga + gb * (double)y;
           NewtonState w{guess, 0., 1., 0};
           if (guess == guess) {
-            newton_resume<N>(P, nw, w, akS, rkS, WARM_MAX_IT);
+            newton_resume<N, false>(P, nw, w, akS, rkS, WARM_MAX_IT);
             total += w.it;
           }
           if (guess == guess && fabs(w.f) <= 1e-10) {
@@ -1073,7 +1073,7 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
         }
         if (!conv) {
           const int before = nst.it;
-          newton_resume<N>(P, nw, nst, akS, rkS, 100);
+          newton_resume<N, false>(P, nw, nst, akS, rkS, 100);
           total += nst.it - before;
           conv = nst.it < 100;
         }
