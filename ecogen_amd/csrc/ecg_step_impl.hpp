@@ -309,21 +309,30 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
       lg = P.lim[0]; lvf = P.lim[2];
     }
   }
-  R lim[(MODEL == M_EULER ? 2 : 3 * N) + D];
+  // All the variables' limited slopes together, except in the three-phase kernels with the kind
+  // fixed at compile time, where each waits until it is used: together they cost the 3D
+  // second-order FP32 kernels 4-5 VGPRs more than the 128 of four waves (93 x 95 x 91, us a step
+  // together / apart: FP64 671 / 639, FP32 244 / 239; two phases 119 x 113 x 117 FP32 330 / 334).
+  constexpr bool LATE = LK >= 0 && N == 3;
+  constexpr int NL = (MODEL == M_EULER ? 2 : 3 * N) + D;
+  R lim[NL];
   if constexpr (LK < 0) {
     if (MODEL != M_EULER) limit_slopes<MODEL, N, D, R, S, true>(lvf, s1, s2, lim);
     limit_slopes<MODEL, N, D, R, S, false>(lg, s1, s2, lim);
-  } else {
+  } else if constexpr (!LATE) {
 #pragma unroll
-    for (int v = 0; v < (MODEL == M_EULER ? 2 : 3 * N) + D; v++) lim[v] = limit<R>(LK, s1[S * v], s2[S * v]);
+    for (int v = 0; v < NL; v++) lim[v] = limit<R>(LK, s1[S * v], s2[S * v]);
   }
+  auto late = [&](int v) {
+    if constexpr (LATE) lim[v] = limit<R>(LK, s1[S * v], s2[S * v]);
+  };
   int v = 0;
 #pragma unroll
   for (int k = 0; k < N; k++) {
     R la = R(0.), lr, lp;
-    if (MODEL != M_EULER) { la = lim[v]; v++; }
-    lr = lim[v]; v++;
-    lp = lim[v]; v++;
+    if (MODEL != M_EULER) { late(v); la = lim[v]; v++; }
+    late(v); lr = lim[v]; v++;
+    late(v); lp = lim[v]; v++;
     if (negate) { la = -la; lr = -lr; lp = -lp; }
     if (MODEL != M_EULER) b.a[k] += la * dist;
     b.r[k] += lr * dist;
@@ -331,6 +340,7 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
     if (MODEL == M_EULER) {
 #pragma unroll
       for (int d = 0; d < D; d++) {
+        late(v + d);
         R lu = lim[v + d];
         if (negate) lu = lu * R(-1.);
         b.u[d] = b.u[d] + lu * dist;
@@ -341,6 +351,7 @@ __device__ __forceinline__ void extrapolate(const Params& P, Cell<N, R>& b, cons
   if (MODEL != M_EULER) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
+      late(v + d);
       R lu = lim[v + d];
       if (negate) lu = lu * R(-1.);
       b.u[d] = b.u[d] + lu * dist;

@@ -62,9 +62,11 @@ def _step(model, nph, dim, second, real, learned, limiter, capture=False, tile=N
             f"ELi{tile}EE")
 
 
-UEQ = 2
-# Finite-rate two-phase 3D FP64: f' in a copy of its own, 41 spills.
-BOUNDS = [(_step(UEQ, 2, 3, False, "d", False, -2), 48)]
+PUEQ, UEQ, MINMOD = 1, 2, 1
+# Second-order three-phase FP32 kernels with the limiter fixed hold each limited slope only
+# where it is used: no scratch.  Finite-rate two-phase 3D FP64: f' in a copy of its own, 41 spills.
+BOUNDS = [(_step(m, 3, 3, True, "f", learned, MINMOD), 0) for m in (PUEQ, UEQ) for learned in (False, True)] + \
+         [(_step(UEQ, 2, 3, False, "d", False, -2), 48)]
 
 
 @pytest.mark.parametrize("name,spills", BOUNDS)
@@ -72,3 +74,5 @@ def test_spilled_registers(kernels, name, spills):
     match = [k for n, k in kernels.items() if name in n]
     assert len(match) == 1, (name, len(match))
     assert match[0][".vgpr_spill_count"] <= spills
+    if spills == 0:
+        assert match[0][".private_segment_fixed_size"] == 0
