@@ -1245,21 +1245,23 @@ __global__ __launch_bounds__(256) void k_fill(Params P, const DomainDev* __restr
   store_prim<MODEL, N, D>(P, W, c, s);
 }
 
-// The small tiles serve meshes whose ordinary tiles leave most of the chip's 256 CUs
-// empty, where a stage lasts as long as one block: up to 256 ordinary tiles at second order
-// in 2D and in FP32, up to 128 at first order and in 3D FP64, where a block's chain is
-// shorter against the small tiles' extra faces.  Both sides measured, a step on caller
-// buffers, ordinary / small tiles (us): 2D two-phase O2 FP64 96^2 90/63, 256^2 87/86, 304^2
-// 93/95, FP32 256^2 71/63; 3D two-phase O2 FP32 32^3 79/63, 44^3 91/107; 2D O1 FP64 160^2
-// 50/46, 256^2 52/55; 3D two-phase O2 FP64 24^3 109/67, 32^3 103/91, 40^3 111/137; Euler
-// O2 FP64 32^3 69/53, 48^3 78/91.  The full-featured and the capture kernels keep the
-// ordinary tiles (their code is long; Euler's LK_FULL, the second-order walls, is the
-// exception).
+// The small tiles serve meshes of at most one ordinary tile per CU, where a stage lasts as
+// long as one block: up to 256 ordinary tiles at second order in 2D and in cold FP32, up to 128 at
+// first order, in 3D FP64 and in the learned 3D kernels, where a block's chain is shorter against
+// the small tiles' extra faces and the inferences of four times the blocks.  Both sides measured, a
+// step of a run, ordinary / small tiles (us).  Two phases: 2D O2 FP64 96^2 110/66, 256^2 89/86, FP32
+// 256^2 124/95; 2D O1 FP64 160^2 48/35, 256^2 40/39; 3D O2 FP32 32^3 112/78, 40^3 (300 tiles) 117/105,
+// FP64 24^3 138/73, 32^3 128/115, 40^3 131/158; 3D O1 FP64 32^3 31/26, 36^3 30/33, FP32 36^3 24/22;
+// learned 3D O2 32^3 54/42, 36^3 (243 tiles) 54/59, 40^3 59/71, O1 36^3 26/34.  Three phases: 2D O2
+// FP64 256^2 94/86; 3D O1 FP64 32^3 34/34, 40^3 56/67; 3D O2 FP64 36^3 206/155, FP32 40^3 176/117;
+// learned 3D O2 36^3 62/68.  Euler: 3D O2 FP64 32^3 37/22, 48^3 78/91.  The full-featured and the
+// capture kernels keep the ordinary tiles (their code is long; Euler's LK_FULL, the second-order
+// walls, is the exception).
 template <int MODEL, int D, int LK, bool CAP> constexpr bool has_small() {
   return D >= 2 && !CAP && (LK != LK_FULL || MODEL == M_EULER);
 }
-template <int D, bool O2, int ES> inline bool step_small(const Params& P) {
-  return (int64_t)P.tiles[0] * P.tiles[1] * P.tiles[2] <= ((O2 && (D == 2 || ES == 4)) ? 256 : 128);
+template <int D, bool O2, int ES, bool LEARN> inline bool step_small(const Params& P) {
+  return (int64_t)P.tiles[0] * P.tiles[1] * P.tiles[2] <= ((O2 && (D == 2 || (ES == 4 && !LEARN))) ? 256 : 128);
 }
 
 // One stage of the step.  The FP32 kernels address the state by 32-bit byte
@@ -1271,7 +1273,7 @@ template <int MODEL, int N, int D, bool O2, typename R, bool LEARN, int LK, bool
 void launch_step_v(const Params& P, const StepLaunchT<R>& L, Clock* clk, Counters* cnt, hipStream_t s) {
   constexpr int ES = (int)sizeof(R);
   if constexpr (!tile_small(TK) && has_small<MODEL, D, LK, CAP>()) {
-    if (step_small<D, O2, ES>(P)) {
+    if (step_small<D, O2, ES, LEARN>(P)) {
       launch_step_v<MODEL, N, D, O2, R, LEARN, LK, CAP, TK + SMALL_TILE>(P, L, clk, cnt, s);
       return;
     }
