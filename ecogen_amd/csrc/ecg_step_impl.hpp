@@ -922,8 +922,14 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
   }
   ConsAcc<N, R> acc;
 
+  // The accumulators' slots lie behind the staging.  They are read back without a barrier
+  // before the inference, whose rows of another wave start at offset 0.
   constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK>();
-  double* st = reinterpret_cast<double*>(lds + Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) + tid;
+  constexpr int STAGED = (int)sizeof(R) * Sizes<MODEL, N, D>::template lds_elems<TK>(O2);
+  static_assert(ST >= 0, "the staging leaves no room for the accumulators");
+  static_assert(ST == 0 || STAGED % 8 == 0, "the accumulators' slots are doubles");
+  static_assert(!LEARN || ST == 0 || STAGED >= step_block_lds<TK>(), "the inference overwrites waiting accumulators");
+  double* st = reinterpret_cast<double*>(lds_raw + STAGED) + tid;
   if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { st[256 * v] = x; });
   if constexpr (tile_small(TK)) {
     // Waves 0-1 take the x axis, 2-3 y, 4-5 z; the first wave gathers in the faces' order.
