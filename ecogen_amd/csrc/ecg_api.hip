@@ -1342,7 +1342,7 @@ int ecg_step_noalloc(const ecg_config* cfg, const void* state_in, void* state_ou
   };
   const size_t o_par = take(sizeof(Params)), o_clk = take(sizeof(Clock));
   const size_t o_cnt = take(sizeof(Counters) * ATOMIC_SLOTS), o_wc = take(sizeof(unsigned long long));
-  // Nine doubles per face of an axis' line that nothing reads: they are part of the size
+  // Three doubles per face of an axis' line that nothing reads: they are part of the size
   // above which a case is refused.
   size_t nface = 0;
   for (int n : {g.nx, g.ny, g.nz}) nface += (size_t)std::max(n - 1, 1);

@@ -468,9 +468,9 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
 // three-phase FP64 kernels need 187 (first order) and 195 registers and have 168 (three
 // waves per SIMD); what a third of a CU's LDS holds beside the staging, seven and six
 // doubles a thread (nine in 2D), takes the accumulators out of the flux passes, where they had been
-// spilled and reloaded in every pass (256^3 first order: 3186 -> 2692 us a step; two waves
-// per SIMD without spills: 3242).  The first-order FP32 kernel runs five waves that way
-// (step_waves).
+// spilled and reloaded in every pass (256^3 first order: 3186 -> 2657 us a step; two waves
+// per SIMD without spills: 3242).  18 (VELOCITYEQ) or 32 VGPRs (Kapila) at first order and 38 to 90 at second
+// order still spill.  The first-order FP32 kernel runs five waves that way (step_waves).
 template <int MODEL, int N, int D, bool O2, int TK, int LK> constexpr int acc_stash() {
   if (!(N == 3 && D >= 2 && (TK == 8 || (TK == 4 && !O2)) && LK != LK_FULL)) return 0;
   const int room = ((TK == 8 ? 53760 : 32256) - TK * Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) / (256 * 8);
