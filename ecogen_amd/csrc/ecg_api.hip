@@ -1042,7 +1042,8 @@ int ecg_run(ecg_ctx* c, int64_t max_iter, double t_end, ecg_step_stats* st) {
 int ecg_tile_of_block(const ecg_config* cfg, int ntiles, int block) {
   if (!cfg || ntiles < 1 || block < 0 || block >= ntiles) return fail(ECG_E_ARG, "block outside the launch");
   const int d = (cfg->nx > 1) + (cfg->ny > 1) + (cfg->nz > 1);
-  return xcd_tile(ntiles, block, tile_run(cfg->model, cfg->nph, d, cfg->precision == ECG_FP32_LEARNED, ntiles));
+  const int esize = cfg->precision == ECG_FP64 ? 8 : 4;
+  return xcd_tile(ntiles, block, tile_run(cfg->model, cfg->nph, d, esize, cfg->precision == ECG_FP32_LEARNED, ntiles));
 }
 
 double ecg_exp(double x) { return exp_cr(x); }

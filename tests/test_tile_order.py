@@ -47,9 +47,10 @@ def test_two_phase_steps_share_any_part_of_the_mesh(model, dim, ntiles):
 
 
 @pytest.mark.parametrize("cfg", [("euler", 1, 2), ("euler", 1, 3), ("pueq", 3, 2), ("ueq", 3, 3), ("pueq", 2, 1),
-                                 ("ueq", 2, 3, "fp32_learned")])
+                                 ("ueq", 2, 3, "fp32_learned"), ("pueq", 2, 2, "fp32", 16383), ("ueq", 2, 3, "fp64", 6145)])
 def test_other_steps_keep_one_range_per_xcd(cfg):
-    for ntiles in (900, 1892, 4375):
+    *cfg, count = cfg if len(cfg) == 5 else (*cfg, 0)
+    for ntiles in (count,) if count else (900, 1892, 4375):
         tile = _order(_config(*cfg), ntiles)
         for x in range(8):
             mine = tile[x::8]
