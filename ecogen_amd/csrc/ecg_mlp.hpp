@@ -250,8 +250,7 @@ __device__ __forceinline__ void mlp_infer_tile(const MlpDev& M, const unsigned s
 // (MLP_WAVE_LDS bytes at lds), and it runs as many 16-row tiles as they fill: a
 // wave without a candidate does nothing, and no other wave is waited for.  The
 // region must be free of other use: the step kernel calls it after its last flux
-// pass, whose closing barrier has released the staging LDS (the accumulators that wait
-// behind the staging are beyond every wave's region).
+// pass, whose closing barrier has released the staging LDS.
 __device__ __forceinline__ float mlp_wave_infer(const MlpDev& M, bool need, const float* x, unsigned char* lds) {
   const int lane = threadIdx.x & 63;
   const unsigned long long m = __ballot(need);

@@ -470,9 +470,11 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
 // doubles a thread (nine in 2D), takes the accumulators out of the flux passes, where they had been
 // spilled and reloaded in every pass (256^3 first order: 3186 -> 2657 us a step; two waves
 // per SIMD without spills: 3242).  18 (VELOCITYEQ) or 32 VGPRs (Kapila) at first order and 38 to 90 at second
-// order still spill.  The first-order FP32 kernel runs five waves that way (step_waves).
-template <int MODEL, int N, int D, bool O2, int TK, int LK> constexpr int acc_stash() {
-  if (!(N == 3 && D >= 2 && (TK == 8 || (TK == 4 && !O2)) && LK != LK_FULL)) return 0;
+// order still spill.  The cold first-order FP32 kernel runs five waves that way (step_waves); the
+// learned one gains no wave, runs 2 % faster without (256^3 13.73 -> 14.01 Gcell-updates/s), and its
+// inference, whose rows start at offset 0 of the LDS, then meets no waiting accumulators.
+template <int MODEL, int N, int D, bool O2, int TK, int LK, bool LEARN> constexpr int acc_stash() {
+  if (LEARN || !(N == 3 && D >= 2 && (TK == 8 || (TK == 4 && !O2)) && LK != LK_FULL)) return 0;
   const int room = ((TK == 8 ? 53760 : 32256) - TK * Sizes<MODEL, N, D>::template lds_elems<TK>(O2)) / (256 * 8);
   return room < 3 * N ? room : 3 * N;
 }
@@ -490,7 +492,7 @@ template <int NS, int N, typename R, class F> __device__ __forceinline__ void ea
 // batches of lines when the staging would exceed lds_batch_bytes.  The small tiles call
 // one step at a time (STEPS) on the axis's own threads, with the barriers between them.
 constexpr int STEP_A = 1, STEP_B = 2, STEP_C = 4, STEP_ABC = 7;
-template <int MODEL, int N, int D, bool O2, typename R, int LK, int AX, int FR, int TK = (int)sizeof(R), int STEPS = STEP_ABC>
+template <int MODEL, int N, int D, bool O2, typename R, int LK, int AX, int FR, bool LEARN, int TK = (int)sizeof(R), int STEPS = STEP_ABC>
 __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>& L, R* lds, const int org[3],
                                           const int own[3], bool own_ok, const R* an, const R* pn, R& smax,
                                           ConsAcc<N, R>& acc) {
@@ -627,7 +629,7 @@ __device__ __forceinline__ void axis_pass(const Params& P, const StepLaunchT<R>&
     if (STEPS == STEP_ABC) __syncthreads();
 
     // C. gather: add the lower face, subtract the upper face
-    constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK>();
+    constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK, LEARN>();
     double* st = reinterpret_cast<double*>(lds + SZ::template lds_elems<TK>(O2)) + threadIdx.x;
     if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { x = st[256 * v]; });
     if ((STEPS & STEP_C) && own_ok && lown / LB == bt) {
@@ -922,13 +924,13 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
   }
   ConsAcc<N, R> acc;
 
-  // The accumulators' slots lie behind the staging.  They are read back without a barrier
-  // before the inference, whose rows of another wave start at offset 0.
-  constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK>();
+  // The accumulators' slots lie behind the staging.  They are read back without a barrier, so
+  // nothing may write LDS after the passes (the learned kernels' inference does).
+  constexpr int ST = acc_stash<MODEL, N, D, O2, TK, LK, LEARN>();
   constexpr int STAGED = (int)sizeof(R) * Sizes<MODEL, N, D>::template lds_elems<TK>(O2);
   static_assert(ST >= 0, "the staging leaves no room for the accumulators");
   static_assert(ST == 0 || STAGED % 8 == 0, "the accumulators' slots are doubles");
-  static_assert(!LEARN || ST == 0 || STAGED >= step_block_lds<TK>(), "the inference overwrites waiting accumulators");
+  static_assert(!LEARN || ST == 0, "the inference would write where accumulators may wait");
   double* st = reinterpret_cast<double*>(lds_raw + STAGED) + tid;
   if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { st[256 * v] = x; });
   if constexpr (tile_small(TK)) {
@@ -936,22 +938,22 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
     const int grp = __builtin_amdgcn_readfirstlane(tid / pass_threads<TK>());
 #define ECG_AXES(STEP)                                                                                               \
   do {                                                                                                               \
-    if (grp == 0) axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
-    else if (grp == 1) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
-    else if constexpr (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
+    if (grp == 0) axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, LEARN, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
+    else if (grp == 1) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, LEARN, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
+    else if constexpr (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, LEARN, TK, STEP>(P, L, lds, org, own, own_ok, an, pn, smax, acc); \
     __syncthreads();                                                                                                 \
   } while (0)
     if constexpr (O2) ECG_AXES(STEP_A);
     ECG_AXES(STEP_B);
 #undef ECG_AXES
-    axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
-    axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
-    if constexpr (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, LEARN, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, LEARN, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    if constexpr (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, LEARN, TK, STEP_C>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
     __syncthreads();
   } else {
-    axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
-    if (D >= 2) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
-    if (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    axis_pass<MODEL, N, D, O2, R, LK, 0, FR_XI, LEARN>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    if (D >= 2) axis_pass<MODEL, N, D, O2, R, LK, 1, FR_YI, LEARN>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
+    if (D >= 3) axis_pass<MODEL, N, D, O2, R, LK, 2, FR_ZI, LEARN>(P, L, lds, org, own, own_ok, an, pn, smax, acc);
   }
   if constexpr (ST > 0) each_stashed<ST, N, R>(acc, [&](double& x, int v) { x = st[256 * v]; });
 
@@ -1297,7 +1299,7 @@ void launch_step_v(const Params& P, const StepLaunchT<R>& L, Clock* clk, Counter
     chunk = (int)std::min<int64_t>(rows, std::max<int64_t>((lines - 4) / T, 1));
     if (chunk < rows && chunk > 1) chunk &= ~1;
   }
-  size_t lds = sizeof(R) * SZ::template lds_elems<TK>(O2) + 256 * sizeof(double) * acc_stash<MODEL, N, D, O2, TK, LK>();
+  size_t lds = sizeof(R) * SZ::template lds_elems<TK>(O2) + 256 * sizeof(double) * acc_stash<MODEL, N, D, O2, TK, LK, LEARN>();
   if (LEARN && lds < (size_t)step_block_lds<TK>()) lds = step_block_lds<TK>();
   auto k = k_step<MODEL, N, D, O2, R, LEARN, LK, CAP, TK>;
   // A failure here surfaces as the launch error the caller checks next.
