@@ -221,7 +221,9 @@ int64_t ecg_ncell(const ecg_ctx* ctx);
  * (Run.cpp:128-140).  Runs on the device. */
 int ecg_fill(ecg_ctx* ctx, const ecg_domain* doms, int ndom);
 
-/* State transfer, host SoA double arrays (layout above). soa[v] points at ncell doubles. */
+/* State transfer, host SoA double arrays (layout above). soa[v] points at ncell doubles.
+ * Downloaded arrays may share memory: the later variable's values then stand.  The first download
+ * allocates up to 8 MB of page-locked memory, freed by ecg_destroy; it works without, more slowly. */
 int ecg_upload_state(ecg_ctx* ctx, const double* const* soa, int nvars);
 int ecg_download_state(ecg_ctx* ctx, double* const* soa, int nvars);
 
