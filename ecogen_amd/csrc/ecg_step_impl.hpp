@@ -441,9 +441,13 @@ __device__ __forceinline__ void tile_origin(const Params& P, int row0, int nrows
   const int t0 = (D == 1) ? nrows : tile_small(TK) ? (P.nx + Tile<D, TK>::X - 1) / Tile<D, TK>::X : P.tiles[0];
   const int t1 = (D == 2) ? nrows : (D == 3) ? tiles1 : 1;
   const int nb = t0 * t1 * ((D == 3) ? nrows : 1);
-  constexpr int ES = tile_esize(TK), RUN = tile_small(TK) ? 0 : tile_run(MODEL, N, D, ES, LEARN, 0);   // of launches in runs
-  const int b = (RUN > 0 && tile_run(MODEL, N, D, ES, LEARN, nb) > 0) ? xcd_tile(nb, blockIdx.x, RUN)
-                                                                      : xcd_tile(nb, blockIdx.x, 0);
+  // The rule's runs as constants, so that the order takes shifts.
+  constexpr int RUN = tile_small(TK) ? 0 : tile_run(MODEL, N, D, tile_esize(TK), LEARN, 4096);
+  constexpr int FEW = tile_small(TK) ? 0 : tile_run(MODEL, N, D, tile_esize(TK), LEARN, 1);
+  const int run = tile_run(MODEL, N, D, tile_esize(TK), LEARN, nb);
+  const int b = (RUN > 0 && run == RUN)   ? xcd_tile(nb, blockIdx.x, RUN)
+                : (FEW > 0 && run == FEW) ? xcd_tile(nb, blockIdx.x, FEW)
+                                          : xcd_tile(nb, blockIdx.x, 0);
   int tx = b % t0;
   const int rest = b / t0;
   int ty = rest % t1;
