@@ -81,18 +81,20 @@ __host__ __device__ inline int xcd_tile(int nb, int block, int run) {
 }
 
 // Tiles per run of xcd_tile for a step launch over nb tiles of 256 cells, of a case with n phases
-// in d dimensions and a state of esize bytes an element; 0: one range per XCD.  Ranges share the most halos, and where every tile costs
-// the same they are the fastest: Euler 3D O1 FP64 at 121 x 119 x 117 97 us a step, dealt singly 157.
+// in d dimensions and a state of esize bytes an element; 0: one range per XCD.  Ranges share the
+// most halos, and where every tile costs the same they are the fastest: Euler 3D O1 FP64 at
+// 121 x 119 x 117 97 us a step, dealt singly 157.
 // A two-phase step's relaxation makes the tiles around a shock and the interfaces cost a multiple
 // of the others, and ranges leave them to one or two XCDs: 2D O1 FP64 at 701 x 683 (1892 tiles) 73
 // us in ranges, 64 dealt singly, 62 in runs of 32 (2048^2 379 / 363 / 367); O2 FP32 113 / 110 / 99
 // (1361 x 1283 233 / 281 / 213; beyond 8192 tiles FP32 ranges win: 2048^2 O1 196 us, in runs 201).
-// Below 512 tiles runs of 16 (208^2, 169 tiles, O1 FP64 48.5 in ranges, 46.3).  In 3D runs of 64 keep the x and y neighbours together: O2 FP64
-// at 93 x 95 x 91 449 / 472 / 423, FP32 222 / 239 / 204; beyond 6144 tiles (eight rounds of three
-// blocks a CU) the costs even out within a range, and its shared z halos win (O1 FP32 at 119 x
-// 113 x 117 144 us, in runs of 64 150).  Three-phase steps gain nothing (2D O1 FP64 at 907 x 883
-// 109 us in ranges and in runs), nor do learned ones in 3D, whose relaxations are short (O1 at 101 x
-// 99 x 97 112 us in ranges, 122 in runs of 32), nor the small tiles, all resident at once.
+// Below 512 tiles runs of 16 (208^2, 169 tiles, O1 FP64 48.5 us in ranges, 46.3).  In 3D runs of
+// 64 keep the x and y neighbours together: O2 FP64 at 93 x 95 x 91 449 / 472 / 423, FP32 222 / 239 /
+// 204; beyond 6144 tiles (eight rounds of three blocks a CU) the costs even out within a range, and
+// its shared z halos win (O1 FP32 at 119 x 113 x 117 144 us, in runs of 64 150).  Three-phase steps
+// gain nothing (2D O1 FP64 at 907 x 883 109 us in ranges and in runs), nor do learned ones in 3D,
+// whose relaxations are short (O1 at 101 x 99 x 97 112 us in ranges, 122 in runs of 32), nor the
+// small tiles, all resident at once.
 __host__ __device__ constexpr int tile_run(int model, int n, int d, int esize, bool learned, int nb) {
   if (model == M_EULER || n != 2 || d == 1) return 0;
   if (d == 2) return nb < 512 ? 16 : esize == 8 || nb <= 8192 ? 32 : 0;
