@@ -209,12 +209,18 @@ __device__ __forceinline__ double div_ieee(double a, double b, double rb) {
 }
 // A single quotient by the same sequence (no pre-scaling and fix-up steps).
 __device__ __forceinline__ double div1(double a, double b) { return div_ieee(a, b, rcp_ieee(b)); }
+// The same with the hardware's fix-up, which gives the special values of zero, infinite and NaN
+// operands: for the quotients whose operands a broken state reaches (its cells are reported, and
+// what it leaves in their neighbours follows the IEEE quotient).
+__device__ __forceinline__ double div_special(double a, double b, double rb) {
+  return __builtin_amdgcn_div_fixup(div_ieee(a, b, rb), b, a);
+}
 // Quotients by one divisor.
 template <typename R> struct Quot;
 template <> struct Quot<double> {
   double b, rb;
   __device__ __forceinline__ explicit Quot(double d) : b(d), rb(rcp_ieee(d)) {}
-  __device__ __forceinline__ double operator()(double a) const { return div_ieee(a, b, rb); }
+  __device__ __forceinline__ double operator()(double a) const { return div_special(a, b, rb); }
 };
 template <> struct Quot<float> {
   float rb;
@@ -228,7 +234,7 @@ struct QuotFull {
   double s, b, rb;
   __device__ __forceinline__ explicit QuotFull(double d) : s(fabs(d) < 1.e-290 ? 0x1p512 : 1.), b(d * s), rb(rcp_ieee(b)) {}
   __device__ __forceinline__ double operator()(double a) const {
-    return __builtin_amdgcn_div_fixup(div_ieee(a, b, rb), b, a) * s;
+    return div_special(a, b, rb) * s;
   }
 };
 // The square root as the device's sequence forms it (reciprocal square-root
@@ -465,11 +471,11 @@ __device__ __forceinline__ R limit(int kind, R s1, R s2) {
   } else if (kind == LIM_VANLEER) {
     R sum = s1 + s2;
     // The quotient always, then a select: no mask and branch around every variable's.
-    const R q = qdiv(R(2.) * prod, sum);
+    const R q = Quot<R>(sum)(R(2.) * prod);
     out = ((fabs(sum) > R(1e-6)) && (prod > R(1e-6))) ? q : R(0.);
   } else if (kind == LIM_VANALBADA) {
     R sum = s1 + s2;
-    const R q = qdiv(prod * sum, s1 * s1 + s2 * s2);
+    const R q = Quot<R>(s1 * s1 + s2 * s2)(prod * sum);
     out = ((fabs(s1) > R(1e-6)) && (fabs(s2) > R(1e-6)) && (fabs(sum) > R(1e-6)) && (prod > R(1e-6))) ? q : R(0.);
   } else if (kind == LIM_SUPERBEE) {
     if (prod > R(1e-6)) out = dmax<R>(dmin<R>(R(2.) * fabs(s1), fabs(s2)), dmin<R>(fabs(s1), R(2.) * fabs(s2)));
@@ -1264,7 +1270,7 @@ __device__ __forceinline__ void build_prim(const Params& P, Cons<N>& A, Cell<N>&
   // Of the derived state only the mixture density is read afterwards (energy
   // correction); the rest is rebuilt from the stored primitives when needed.
   mixture_density<N>(s);
-  s.E = div_ieee(A.energM, rhoMel, irm);
+  s.E = div_special(A.energM, rhoMel, irm);
 }
 
 // alphaNull gate of RelaxationPInfinite::relaxation (RelaxationPInfinite.cpp:51-55):
@@ -1583,7 +1589,7 @@ __device__ __forceinline__ void correct_and_derive(const Params& P, Cell<N>& s) 
       pp -= s.a[k] * (P.eos[k].mixg * (1. - s.r[k] * 0.) + s.r[k] * P.eos[k].eref);
       denom += s.a[k] * P.eos[k].mixinv * (1. - s.r[k] * 0.);
     }
-    pp = div1(pp, denom);
+    pp = div_special(pp, denom, rcp_ieee(denom));
 #pragma unroll
     for (int k = 0; k < N; k++) {
       s.p[k] = pp;

@@ -1010,7 +1010,7 @@ __global__ __launch_bounds__((tile_threads<D, TK>()), (step_waves<R, N, D, O2, L
       for (int k = 0; k < N; k++) un += own64.a[k];
       const double iun = rcp_ieee(un);
 #pragma unroll
-      for (int k = 0; k < N; k++) own64.a[k] = div_ieee(own64.a[k], un, iun);
+      for (int k = 0; k < N; k++) own64.a[k] = div_special(own64.a[k], un, iun);
     }
     // U^n needs the mixture density of the time-n cell (Cell::timeEvolution rebuilds
     // the conservative variables from the primitives, FluxUEq::buildCons).
