@@ -582,14 +582,15 @@ __device__ __forceinline__ void derive(const Params& P, Cell<N, R>& s, bool rebu
     if constexpr (sizeof(R) == 8) {
       // One reciprocal of the density for the energy and the squared sound speed.  Euler
       // densities and pressures carry no floor: a vacuum's sound speed is infinite, which makes the
-      // step's dtMax zero, so the hardware's fix-up gives the quotient by a zero density (one whose
-      // reciprocal overflows counts as zero) and the library's root the special values.  (The
-      // lean root with a test of its range before the library's: 121 x 119 x 117 first order 96
-      // us a step, this 88; with second-order walls 357 / 343.)
+      // step's dtMax zero, so the hardware's fix-up gives the quotient by a zero density and the
+      // library's root the special values.  (The lean root with a test of its range before the
+      // library's: 121 x 119 x 117 first order 96 us a step, this 88; with second-order walls
+      // 357 / 343.)  The fix-up's divisor is scaled so that a density whose reciprocal overflows
+      // rounds to the zero of its sign (-0 has no sound speed, as in the reference).
       const EosDev& q = P.eos[0];
       const double rr = dmax<double>(s.r[0], eps), ir = rcp_ieee(rr), cn = q.g * (s.p[0] + q.pinf);
       s.e[0] = div_ieee(div_ieee(s.p[0] + q.gpinf, q.gm1, q.mixinv), rr, ir) + q.eref;
-      s.c[0] = sqrt(__builtin_amdgcn_div_fixup(div_ieee(cn, rr, ir), rr < 0x1p-1024 ? 0. : rr, cn));
+      s.c[0] = sqrt(__builtin_amdgcn_div_fixup(div_ieee(cn, rr, ir), rr * 0x1p-51, cn));
     } else {
       s.e[0] = eos_energy<R>(P.eos[0], eps, s.r[0], s.p[0]);
       s.c[0] = eos_sound<R>(P.eos[0], eps, s.r[0], s.p[0]);

@@ -1,5 +1,5 @@
-"""Euler cells of zero, negative and subnormal density or of zero and negative pressure, whose
-densities and pressures the model does not floor, against the oracle (needs a GPU): the same
+"""Euler cells of zero (of either sign), negative and subnormal density or of zero and negative
+pressure, whose densities and pressures the model does not floor, against the oracle (needs a GPU): the same
 dtMax (a vacuum's infinite sound speed makes it zero), the same cells left non-finite, an error
 exactly when there are any, and the other cells within the parity bar of 1e-12."""
 import ctypes as C
@@ -9,7 +9,8 @@ import pytest
 
 from ecogen_amd.case import sod_case
 
-CELLS = {"vacuum": (20, 0., 1.e5, 0.), "negative_density": (20, -1.e-3, 1.e5, 0.), "empty": (20, 0., 0., 0.),
+CELLS = {"vacuum": (20, 0., 1.e5, 0.), "negative_zero_density": (20, -0., 1.e5, 0.),
+         "negative_density": (20, -1.e-3, 1.e5, 0.), "empty": (20, 0., 0., 0.),
          "no_pressure": (20, 1., 0., 0.), "tension": (20, 1., -1., 0.), "subnormal_density": (20, 1.e-310, 1.e5, 0.),
          "vacuum_at_the_end": (63, 0., 1.e5, 0.), "vacuum_in_supersonic_flow": (20, 0., 1.e5, 2000.)}
 
